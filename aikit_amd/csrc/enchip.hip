@@ -22,6 +22,7 @@
 #include "encoder_ops.h"
 #include "gemm_f32.h"
 #include "gemm_persistent.h"
+#include "gemm_pieces.h"
 #include "gemm_q8w.h"
 #include "gemm_skinny.h"
 #include "topk.h"
@@ -420,6 +421,41 @@ bool route_af(const enchip_ctx *c, const Weight &w, int64_t M, const void *out, 
     return M > c->small_m && use_persistent(w, nullptr, w.Kp, out, ldo, M, true);
 }
 
+// gemm_pieces.h's piece size for a GEMM on fragment-major codes, as an index into kPieces
+// (-1: gemm_w8a8_pt's or the general kernel's tiles). Pieces pay while their number is a few
+// per CU; past that the larger tiles' fewer loads per output win. Measured on MI355X (graph
+// replay; (M, N, K), 64 x 64 pieces' number, tiles -> pieces): bias only, (512, 4096, 1024),
+// 512: 9.4 -> 8.6 us, (1024, 2304, 768), 576: 7.0 -> 7.6, (1024, 3072, 768), 768: 7.2 -> 8.7.
+// With the GELU, whose VALU work the tiles leave to few wavefronts: (2048, 2304, 768), 1152:
+// 15.1 -> 14.6 at 7% erf tails and 25.3 -> 16.4 at 25%, (2048, 3072, 768), 1536: 15.6 -> 18.3
+// and 26.9 -> 20.1. `ragged`: the outputs gemm_w8a8_pt cannot store, against gemm_w8a8 on
+// row-major codes (linears of N = 1001): (4000, K = 768), 1008 pieces, 22.0 -> 20.5 us, (5000,
+// 384), 1264, 19.6 -> 21.0; with the GELU (5000, 768) 41.8 -> 28.3; (40, 768) 13.5 -> 6.0.
+// Size: 32 x 32 while a CU gets few of them (long K: each wavefront's serial steps are what
+// is left, and larger pieces load less), 64 x 32 for K <= 1024 or few pieces, else 64 x 64:
+// (512, 768, 3072) 5.5 / 4.9 / 6.2 us, (1024, 768, 3072) 7.6 / 7.6 / 6.6, (512, 2304, 768)
+// 5.5 / 5.5 / 6.1, (256, 768, 768) 2.9 / 3.3 / 4.2; with the GELU (1024, 768, 768)
+// 5.4 / 6.2 / 6.9.
+struct Piece {
+    int cm, cn;
+};
+constexpr Piece kPieces[3] = {{32, 32}, {64, 32}, {64, 64}};
+
+int piece_form(const enchip_ctx *c, const Weight &w, int64_t M, int epi, bool ragged) {
+    const int64_t cus = c->num_cus;
+    const bool gelu = epi == enchip::EPI_F32_GELU, short_k = w.Kp <= 1024;
+    auto pieces = [&](int64_t cm, int64_t cn) { return ((M + cm - 1) / cm) * ((w.N + cn - 1) / cn); };
+    if (pieces(64, 64) > (gelu ? 5 : ragged ? 4 : 2) * cus) return -1;
+    if (pieces(32, 32) <= (gelu ? 2 : 1) * (short_k ? 2 : 1) * cus) return 0;
+    return short_k || pieces(64, 32) <= (gelu ? 3 : 1) * cus ? 1 : 2;
+}
+
+// True when a GEMM on codes this library quantizes itself takes them fragment-major: either
+// gemm_w8a8_pt's outputs (route_af, which enchip_frag_route reports), or ragged ones in pieces.
+bool route_frag(const enchip_ctx *c, const Weight &w, int64_t M, int epi, const void *out, int64_t ldo) {
+    return route_af(c, w, M, out, ldo) || (M > c->small_m && piece_form(c, w, M, epi, true) >= 0);
+}
+
 // Small-M kernel choice: gemv_w8a8_wide (one wavefront per 32-channel group, whole K)
 // once there are enough groups to spread over the SIMDs, else gemv_w8a8 (one workgroup
 // per group, K split over its waves). Measured crossover on MI355X (M=1..16): with
@@ -525,7 +561,24 @@ void launch_skinny(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq, int
     else launch_skinny_mb<8, EPI, AF>(c, w, nk, aq, lda, as, bias, out, ldo, M, s, sink);
 }
 
-// af: aq is fragment-major (the caller checked route_af); otherwise row-major at pitch lda.
+// Piece sizes as kPieces. pt: gemm_w8a8_pt's outputs (16-byte stores), else any.
+template <int EPI, int F>
+void launch_pieces(const Weight &w, const int8_t *aq, const float *as, const float *bias, void *out, int64_t ldo,
+                   int64_t M, hipStream_t s, bool pt) {
+    using namespace enchip;
+    constexpr int CM = kPieces[F].cm, CN = kPieces[F].cn;
+    const int64_t pn = (w.N + CN - 1) / CN;
+    const dim3 block(64 * PT_NW);
+    if (pt)
+        hipLaunchKernelGGL((gemm_w8a8_pt<PT_BM_SMALL, PT_BN, PT_BK, PT_PW, EPI, true, PT_NW, 0, CM, CN>),
+                           dim3((unsigned)((M + PT_BM_SMALL - 1) / PT_BM_SMALL * (PT_BM_SMALL / CM) * pn)), block, 0, s, aq,
+                           w.d_w, as, w.d_s, bias, out, ldo, (int)M, (int)w.N, (int)w.Kp, (int)pn);
+    else
+        hipLaunchKernelGGL((gemm_w8a8<CM, CN, EPI, PT_NW, PT_PW>), dim3((unsigned)((M + CM - 1) / CM * pn)), block, 0, s, aq,
+                           w.d_w, as, w.d_s, bias, out, ldo, (int)M, (int)w.N, (int)w.Kp, (int)pn);
+}
+
+// af: aq is fragment-major (the caller checked route_frag); otherwise row-major at pitch lda.
 // Returns false, launching nothing, when the chosen kernel's grid would not fit.
 template <int EPI>
 bool launch_gemm_epi(enchip_ctx *c, const Weight &w, const int8_t *aq, int64_t lda, const float *as,
@@ -536,6 +589,15 @@ bool launch_gemm_epi(enchip_ctx *c, const Weight &w, const int8_t *aq, int64_t l
             else launch_skinny<enchip::EPI_F32, false>(c, w, nk, aq, lda, as, bias, (float *)out, ldo, M, s);
             return true;
         }
+    }
+    if (af) {
+        const bool pt = use_persistent(w, aq, lda, out, ldo, M, true);
+        const int f = piece_form(c, w, M, EPI, !pt);
+        if (f == 0) launch_pieces<EPI, 0>(w, aq, as, bias, out, ldo, M, s, pt);
+        else if (f == 1) launch_pieces<EPI, 1>(w, aq, as, bias, out, ldo, M, s, pt);
+        else if (f == 2) launch_pieces<EPI, 2>(w, aq, as, bias, out, ldo, M, s, pt);
+        else if (!pt) return false;
+        if (f >= 0) return true;
     }
     if (af || (M > c->small_m && use_persistent(w, aq, lda, out, ldo, M, false))) {
         if (af) launch_pt<enchip::PT_PW, EPI, true>(c, w, aq, lda, as, bias, out, ldo, M, s);
@@ -779,9 +841,19 @@ int enchip_gemm_kernel_name(enchip_ctx *ctx, enchip_weight h, int64_t M, int act
     const int sk = epi == enchip::EPI_F32 ? skinny_nk(ctx, *w, M, nullptr, w->Kp, true) : 0;
     if (sk)  // the library's own quantization is fragment-major (pre_dev's row-major codes: false)
         snprintf(name, sizeof name, "enchip::gemm_w8a8_skinny<%d, %d, %d, true>", M <= 128 ? 4 : 8, sk, epi);
-    else if (route_af(ctx, *w, M, nullptr, w->N))
-        snprintf(name, sizeof name, "enchip::gemm_w8a8_pt<%d, %d, %d, %d, %d, true, %d, %d>", pt_bm(ctx, *w, M),
-                 enchip::PT_BN, enchip::PT_BK, pt_ring(*w), epi, enchip::PT_NW, pt_prio(*w, epi));
+    else if (const bool pt = route_af(ctx, *w, M, nullptr, w->N); pt || route_frag(ctx, *w, M, epi, nullptr, w->N)) {
+        const int f = piece_form(ctx, *w, M, epi, !pt);
+        if (f >= 0 && pt)
+            snprintf(name, sizeof name, "enchip::gemm_w8a8_pt<%d, %d, %d, %d, %d, true, %d, 0, %d, %d>",
+                     enchip::PT_BM_SMALL, enchip::PT_BN, enchip::PT_BK, enchip::PT_PW, epi, enchip::PT_NW, kPieces[f].cm,
+                     kPieces[f].cn);
+        else if (f >= 0)
+            snprintf(name, sizeof name, "enchip::gemm_w8a8<%d, %d, %d, %d, %d>", kPieces[f].cm, kPieces[f].cn, epi,
+                     enchip::PT_NW, enchip::PT_PW);
+        else
+            snprintf(name, sizeof name, "enchip::gemm_w8a8_pt<%d, %d, %d, %d, %d, true, %d, %d>", pt_bm(ctx, *w, M),
+                     enchip::PT_BN, enchip::PT_BK, pt_ring(*w), epi, enchip::PT_NW, pt_prio(*w, epi));
+    }
     else if (fused_small_m(ctx, *w, M, nullptr) && epi != enchip::EPI_I32)
         snprintf(name, sizeof name, "enchip::gemv_w8a8_q<%d, %d>", epi, gvq_qch(w->K));
     else if (M <= ctx->small_m && gemv_wide(ctx, *w))
@@ -1211,7 +1283,7 @@ int enchip_w8a8_linear_dev(enchip_ctx *ctx, enchip_weight h, const float *d_a, i
         return launch_fused_small_m(ctx, *w, d_a, M, d_bias, act_code(act), d_dst, w->N, s);
     if ((rc = ensure_act_scratch(ctx, M, w->Kp))) return rc;
     if ((rc = scratch_wait(ctx, s))) return rc;
-    const bool af = route_af(ctx, *w, M, d_dst, w->N);
+    const bool af = route_frag(ctx, *w, M, act_code(act), d_dst, w->N);
     if ((rc = launch_quant(ctx, d_a, M, w->K, ctx->d_aq, w->Kp, ctx->d_as, s, af))) return rc;
     if ((rc = launch_gemm(ctx, *w, ctx->d_aq, w->Kp, ctx->d_as, d_bias, act_code(act), d_dst, w->N, M, s, af)))
         return rc;
@@ -1237,9 +1309,12 @@ int enchip_w8a8_linear_noalloc_dev(enchip_ctx *ctx, enchip_weight h, const float
     }
     if (!ctx->noalloc) return fail(ctx, ENCHIP_ERR_HIP, "linear_noalloc: %s", ctx->noalloc_err.c_str());
     // fragment-major codes are read up to the next multiple of PT_BM rows, row-major
-    // ones up to row M - 1 (the same routes as enchip_w8a8_linear_dev)
-    const bool af = route_af(ctx, *w, M, d_dst, w->N);
-    const int64_t code_bytes = (af ? round_up(M, enchip::PT_BM) : M) * w->Kp;
+    // ones up to row M - 1 (the same routes as enchip_w8a8_linear_dev, except that a ragged
+    // output whose padded codes do not fit stays on the row-major kernel)
+    const int64_t frag_bytes = round_up(M, enchip::PT_BM) * w->Kp;
+    const bool af = route_af(ctx, *w, M, d_dst, w->N) ||
+                    ((size_t)frag_bytes <= kNoAllocCodeBytes && route_frag(ctx, *w, M, act_code(act), d_dst, w->N));
+    const int64_t code_bytes = af ? frag_bytes : M * w->Kp;
     if ((size_t)code_bytes > kNoAllocCodeBytes)
         return fail(ctx, ENCHIP_ERR_ARG, "linear_noalloc: M=%lld x padded K %lld needs %lld code bytes, more than the "
                     "%zu of the no-alloc scratch", (long long)M, (long long)w->Kp, (long long)code_bytes,
@@ -1291,7 +1366,8 @@ int enchip_w8a8_linear(enchip_ctx *ctx, enchip_weight h, const float *a, int64_t
     if ((rc = scratch_wait(ctx, s))) return rc;
     if ((rc = upload(ctx, ctx->d_a, a, (size_t)(M * K) * sizeof(float), s))) return rc;
     if (bias && (rc = upload(ctx, ctx->d_bias, bias, (size_t)N * sizeof(float), s))) return rc;
-    const bool af = route_af(ctx, *w, M, ctx->d_dst, N) && (!acc_debug || route_af(ctx, *w, M, ctx->d_acc, N));
+    const bool af = route_frag(ctx, *w, M, act_code(act), ctx->d_dst, N) &&
+                    (!acc_debug || route_frag(ctx, *w, M, enchip::EPI_I32, ctx->d_acc, N));
     if (!acc_debug && fused_small_m(ctx, *w, M, ctx->d_a)) {
         if ((rc = launch_fused_small_m(ctx, *w, ctx->d_a, M, bias ? ctx->d_bias : nullptr, act_code(act), ctx->d_dst,
                                        N, s)))
@@ -1352,7 +1428,7 @@ int enchip_w8a8_batch(enchip_ctx *ctx, const float *a, int64_t M, int64_t K, con
     // one quantization serves every op, so its layout must suit all of them
     bool af = true;
     for (int i = 0; i < nops; ++i)
-        af = af && route_af(ctx, *ws[(size_t)i], M, ctx->d_dst + dst_off[(size_t)i], ws[(size_t)i]->N);
+        af = af && route_frag(ctx, *ws[(size_t)i], M, act_code(ops[i].act), ctx->d_dst + dst_off[(size_t)i], ws[(size_t)i]->N);
     if ((rc = launch_quant(ctx, ctx->d_a, M, K, ctx->d_aq, Kp, ctx->d_as, s, af))) return rc;
     for (int i = 0; i < nops; ++i) {
         const Weight &w = *ws[(size_t)i];
