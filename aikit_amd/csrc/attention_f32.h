@@ -48,12 +48,6 @@ __host__ __device__ inline int att_lds_floats(int L) {
 constexpr int ATT_QPITCH = 144;  // bytes per Q row per plane (head dim <= 64)
 __host__ __device__ inline int att_split_lds_floats(int L) { return att_lds_floats(L) + 2 * ATT_QT * ATT_QPITCH / 4; }
 
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // 8 consecutive floats from a 16-byte aligned address.
 __device__ __forceinline__ void load8(const float *p, float *d) {
     const f32x4 a = *reinterpret_cast<const f32x4 *>(p), b = *reinterpret_cast<const f32x4 *>(p + 4);
@@ -232,7 +226,6 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 4) void attention_f32(
 // hi plane at byte 0 and a bf16 lo plane at byte 2P + 8 (both 16-byte aligned, 32 * nkt
 // entries each), and each softmax lane owns 2 adjacent columns so that both planes are
 // written a 32-bit word at a time. Non-finite operands give NaN (inf - inf in the split).
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 

@@ -1463,14 +1463,41 @@ int launch_matmul_f32(enchip_ctx *c, const float *A, int64_t lda, const float *B
     if (M == 0 || N == 0 || b1.count == 0 || b2.count == 0) return ENCHIP_OK;
     const F32Strides s1{b1.stride_a, b1.stride_b, b1.stride_c}, s2{b2.stride_a, b2.stride_b, b2.stride_c};
     auto al4 = [](int64_t v) { return v % 4 == 0; };
-    const bool vec = K % 4 == 0 && al4(lda) && al4(s1.a) && al4(s2.a) && (uintptr_t)A % 16 == 0 &&
-                     (bkn || (al4(ldb) && al4(s1.b) && al4(s2.b) && (uintptr_t)B % 16 == 0));
-    const bool km = K % F32_KB != 0;
-    // the LDS-staged kernel loads whole float4 of A rows and of B rows ([N,K]) or B k-rows ([K,N])
-    const bool lds = K % 4 == 0 && al4(lda) && al4(s1.a) && al4(s2.a) && (uintptr_t)A % 16 == 0 && al4(ldb) &&
+    // 16-byte loads: whole float4 of A rows and of B rows ([N,K]) or B k-rows ([K,N])
+    const bool vec = K % 4 == 0 && al4(lda) && al4(s1.a) && al4(s2.a) && (uintptr_t)A % 16 == 0 && al4(ldb) &&
                      al4(s1.b) && al4(s2.b) && (uintptr_t)B % 16 == 0 && (!bkn || N % 4 == 0);
-    const int wm = N <= 64 ? 4 : (M <= 64 ? 1 : 2), wn = 4 / wm;
-    const int tilesM = (int)((M + 64 * wm - 1) / (64 * wm)), tilesN = (int)((N + 64 * wn - 1) / (64 * wn));
+    // The K split (its own summation order, so the choice looks at one problem alone: a batch
+    // gives its problems' bits) for at most 128 tiles of 64 x 64, wide outputs and a long K:
+    // 512 x 768, K = 768 (96 tiles) 12.0 us against 18.1; 512 x 3072 (384) 32.2 against 22.9.
+    // Narrow outputs (scores . V) come in batches, where the tiles are faster: 512 x 64, K =
+    // 512 over 384 heads 142 against 134. Tile sizes, by the launch's number of tiles: the
+    // largest that still give every CU work (the kernels' comments have the figures).
+    const int64_t cus = c->num_cus, nb = b1.count * b2.count;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const bool ksplit = K >= 256 && N > 128 && tiles(64, 64) <= cus / 2;
+    int bm, bn;
+    if (ksplit) {
+        bm = tiles(32, 32) * nb <= cus ? 32 : 64;
+        bn = bm == 32 || tiles(64, 32) * nb <= 2 * cus ? 32 : 64;
+    } else if (M > 64 && N > 64 && tiles(128, 128) * nb >= cus) {
+        bm = bn = 128;
+    } else if (N > 64 && tiles(64, 128) * nb > cus / 2 && tiles(64, 128) * nb <= cus) {
+        bm = 64, bn = 128;
+    } else {
+        bm = tiles(64, 64) * nb > 2 * cus ? 128 : 64, bn = 64;
+    }
+    // Columns per launch: with M * N <= 2^36 every launch's threads then stay below 2^32 (only
+    // M <= 128 has more columns).
+    constexpr int64_t kCols = (int64_t)1 << 28;
+    if (N > kCols) {
+        for (int64_t n0 = 0; n0 < N; n0 += kCols) {
+            const int rc = launch_matmul_f32(c, A, lda, bkn ? B + n0 : B + n0 * ldb, ldb, bkn, C + n0, ldc, M, K,
+                                             std::min(kCols, N - n0), b1, b2, s);
+            if (rc) return rc;
+        }
+        return ENCHIP_OK;
+    }
+    const int64_t tilesN = (N + bn - 1) / bn;
     constexpr int64_t kGrid = 65535;
     for (int64_t z0 = 0; z0 < b2.count; z0 += kGrid)
         for (int64_t y0 = 0; y0 < b1.count; y0 += kGrid) {
@@ -1486,51 +1513,28 @@ int launch_matmul_f32(enchip_ctx *c, const float *A, int64_t lda, const float *B
                 }
                 continue;
             }
-            const dim3 grid((unsigned)(tilesM * tilesN), ny, nz), block(256);
-            if (lds) {
-                if (wm == 4 && bkn)
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<4, 1, true>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1, s2,
-                                       (int)M, (int)N, (int)K, tilesN);
-                else if (wm == 4)
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<4, 1, false>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1,
-                                       s2, (int)M, (int)N, (int)K, tilesN);
-                else if (wm == 1 && bkn)
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<1, 4, true>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1, s2,
-                                       (int)M, (int)N, (int)K, tilesN);
-                else if (wm == 1)
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<1, 4, false>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1,
-                                       s2, (int)M, (int)N, (int)K, tilesN);
-                else if (bkn)
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<2, 2, true>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1, s2,
-                                       (int)M, (int)N, (int)K, tilesN);
-                else
-                    hipLaunchKernelGGL((gemm_f32_bt_lds<2, 2, false>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1,
-                                       s2, (int)M, (int)N, (int)K, tilesN);
-                continue;
-            }
-#define F32_CALL(WM, WN, BKN, VEC, KM)                                                                          \
-    hipLaunchKernelGGL((gemm_f32_bt<WM, WN, BKN, VEC, KM>), grid, block, 0, s, a, lda, b, ldb, cz, ldc, s1, s2,   \
-                       (int)M, (int)N, (int)K, tilesN)
-#define F32_KM(WM, WN, BKN, VEC)                                                                               \
-    do {                                                                                                       \
-        if (km) F32_CALL(WM, WN, BKN, VEC, true);                                                              \
-        else F32_CALL(WM, WN, BKN, VEC, false);                                                                \
+            const dim3 grid((unsigned)tiles(bm, bn), ny, nz);
+#define F32_CALL(KERNEL, THREADS)                                                                             \
+    hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, s, a, lda, b, ldb, cz, ldc, s1, s2, (int)M, (int)N, (int)K, \
+                       (int)tilesN)
+#define F32_LAUNCH(BKN, VEC)                                                                     \
+    do {                                                                                         \
+        if (ksplit && bm == 32) F32_CALL((gemm_f32_ksplit<1, 1, BKN, VEC>), 256);                \
+        else if (ksplit && bn == 32) F32_CALL((gemm_f32_ksplit<2, 1, BKN, VEC>), 256);           \
+        else if (ksplit) F32_CALL((gemm_f32_ksplit<2, 2, BKN, VEC>), 256);                       \
+        else if (bm == 128 && bn == 128) F32_CALL((gemm_f32_tile<2, 2, 2, 2, 16, BKN, VEC>), 256); \
+        else if (bn == 128) F32_CALL((gemm_f32_tile<1, 1, 2, 4, 32, BKN, VEC>), 512);            \
+        else if (bm == 128) F32_CALL((gemm_f32_tile<1, 2, 4, 1, 16, BKN, VEC>), 256);            \
+        else F32_CALL((gemm_f32_tile<1, 1, 2, 2, 32, BKN, VEC>), 256);                           \
     } while (0)
-#define F32_LAUNCH(WM, WN)                                                                                     \
-    do {                                                                                                       \
-        if (bkn && vec) F32_KM(WM, WN, true, true);                                                            \
-        else if (bkn) F32_KM(WM, WN, true, false);                                                             \
-        else if (vec) F32_KM(WM, WN, false, true);                                                             \
-        else F32_KM(WM, WN, false, false);                                                                     \
-    } while (0)
-            if (wm == 4) F32_LAUNCH(4, 1);
-            else if (wm == 1) F32_LAUNCH(1, 4);
-            else F32_LAUNCH(2, 2);
+            if (bkn && vec) F32_LAUNCH(true, true);
+            else if (bkn) F32_LAUNCH(true, false);
+            else if (vec) F32_LAUNCH(false, true);
+            else F32_LAUNCH(false, false);
 #undef F32_CALL
-#undef F32_KM
 #undef F32_LAUNCH
         }
-    return check_launch(c, "gemm_f32_bt");
+    return check_launch(c, "gemm_f32");
 }
 
 constexpr int64_t kMaxDimF32 = (int64_t)1 << 30;  // M, N, K; and M*N below 2^36 elements

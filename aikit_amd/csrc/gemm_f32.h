@@ -1,4 +1,4 @@
-// gemm_f32.h -- f32 C = A . B^T on the gfx950 f32 MFMA: the device side of
+// gemm_f32.h -- f32 C = A . B^T on the gfx950 bf16 MFMA: the device side of
 // encoder.Backend.MatmulBT (encoder/backend.go:19-28), used by attention for
 // QK^T = qH . kH^T and scores . V = scores . (vHT)^T (encoder/attention.go:108,111).
 //
@@ -9,18 +9,30 @@
 // B is [N, K] rows (MatmulBT's b, BKN = false) or [K, N] rows (BKN = true: V itself
 // for scores . V, element (n, k) at B[k*ldb + n], so no transpose copy either).
 //
-// Each wavefront computes a 64 x 64 tile of C as 2 x 2 accumulators of
-// v_mfma_f32_32x32x2_f32. In MFMA step s of a 16-deep K block, lane l supplies
-// row / column l % 32 at k = k0 + 8*(l/32) + s for both operands, so every lane reads
-// 8 consecutive k of its row per block (two 16-byte loads when the rows are 16-byte
-// aligned, VEC). The sum is the exact dot product's terms, each product rounded once
-// and added in f32 in a different order than the CPU's; the contract is the
-// reference's gate against a float64 dot product (gpu/enccuda/backend_test.go:47-86).
-// Two forms with the same k order (so the same bits): gemm_f32_bt_lds stages 16-deep K
-// chunks of the block's operands through LDS with coalesced 16-byte loads (the one used
-// whenever alignment allows), gemm_f32_bt loads each lane's operands straight into
-// registers (any pitch or alignment; latency-bound, about 1.4x slower). Elements past K
-// count as zero; rows past M and columns past N are clamped on load and never stored.
+// Arithmetic. Every operand value is split exactly into three bf16 parts, x = h + m + l (h
+// the bf16 nearest x, m the one nearest x - h, l the rest, which has at most 8 bits), and a
+// product is the six products of parts above 2^-25 of it: h.h', h.m', m.h', m.m', h.l', l.h',
+// each exact on v_mfma_f32_32x32x16_bf16 and summed in f32. The three left out, m.l', l.m'
+// and l.l', are within 2^-26 |x y|, an eighth of what rounding the sum once costs, and a
+// 16-deep step rounds the sum 6 times where the f32 MFMA (32x32x2) rounds it 8 to 16 times.
+// Measured against float64 (standard normal operands, relative 2-norm): K = 768 4.2e-7, or
+// 2.1e-7 with K split over wavefronts, against the f32 MFMA's 5.0e-7; K = 3072 8.7e-7 /
+// 4.3e-7 against 9.9e-7. (Parts below 2^-126 may be flushed: an absolute error under 2^-126
+// times the other operand.) The contract is the reference's gate against a float64 dot
+// product (gpu/enccuda/backend_test.go:47-86).
+// An operand the split cannot hold (an infinity, or a value that rounds to one in bf16) or a
+// sum that overflows leaves a non-finite accumulator; the 32 x 32 blocks of a wavefront that
+// sees one are computed again by f32_block on the f32 MFMA, so infinities and overflow give
+// what f32 arithmetic gives.
+//
+// bf16 products run at 16 times the f32 MFMA's rate, so the six cost 0.38 of it; the f32
+// kernel these replace reached 110-120 of its 154 TFLOP/s at 4096^2 and less than a third of
+// that where its 128 x 128 tiles left CUs idle. Two forms, one result per shape:
+//   gemm_f32_tile  block tiles with the parts staged in LDS;
+//   gemm_f32_ksplit  K split over the wavefronts of small tiles, for shapes with so few
+//                  tiles that the serial K loop is the time.
+// The choice between them depends on M, N and K alone, and each gives the same bits for any
+// tile size, batch, pitch, alignment and layout of the same operands.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -29,297 +41,406 @@
 
 #include "kernels.h"
 
+#pragma clang fp contract(off)
+
 namespace enchip {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int F32_KB = 16;  // K block per pipeline stage
-
-// 8 consecutive k (k0 .. k0+7) of one row, raw: addresses past K are clamped into the
-// row (kmask zeroes those values where they are used). VEC: the row start and k0 are
-// 16-byte aligned and K % 4 == 0, so each float4 is either all in range or all past K.
-template <bool VEC>
-__device__ __forceinline__ void load8_row(const float *__restrict__ row, int k0, int K, float (&v)[8]) {
-    if (VEC) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const f32x4 t = *reinterpret_cast<const f32x4 *>(row + min(k0 + 4 * j, K - 4));
-            v[4 * j + 0] = t.x;
-            v[4 * j + 1] = t.y;
-            v[4 * j + 2] = t.z;
-            v[4 * j + 3] = t.w;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = row[min(k0 + j, K - 1)];
-    }
-}
-
-// 8 consecutive k of column n of a [K, N] matrix (pitch ldb), raw as load8_row.
-__device__ __forceinline__ void load8_col(const float *__restrict__ col, int64_t ldb, int k0, int K, float (&v)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = col[(int64_t)min(k0 + j, K - 1) * ldb];
-}
-
-// Zero the values of k >= K (k0 .. k0+7 held in v).
-__device__ __forceinline__ void kmask(float (&v)[8], int k0, int K) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = k0 + j < K ? v[j] : 0.0f;
-}
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Batch strides of one level (in floats).
 struct F32Strides {
     int64_t a, b, c;
 };
 
-// WM x WN wavefronts per block (block tile 64*WM x 64*WN); grid (tilesM*tilesN, inner
-// batch, outer batch). KM: K is not a multiple of 16, so the last block's k >= K are zeroed.
-template <int WM, int WN, bool BKN, bool VEC, bool KM>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_bt(
+// A workgroup barrier that orders LDS accesses only: global loads in flight stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The three bf16 parts of a (low half) and b (high half of each word).
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+    h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+    m = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
+    const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
+    l = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{sa, sb}), bf16x2));
+}
+
+// acc += the six products of one 16-deep step, smallest first; p[.][0..2] = h, m, l.
+template <int TM, int TN>
+__device__ __forceinline__ void mfma_parts(const bf16x8 (&pa)[TM][3], const bf16x8 (&pb)[TN][3], f32x16 (&acc)[TM][TN]) {
+    constexpr int pi[6] = {2, 0, 1, 1, 0, 0}, qi[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int u = 0; u < 6; ++u)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][pi[u]], pb[t][qi[u]], acc[i][t], 0, 0, 0);
+}
+
+// Whether any accumulator of the lane is infinite or NaN.
+template <int TM, int TN>
+__device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN]) {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s += acc[i][t][e] * 0.0f;
+    return s != 0.0f;  // 0, or NaN
+}
+
+// The 32 x 32 outputs at (m0, n0) of one wavefront on the f32 MFMA, operands loaded value by
+// value: for the rare blocks whose split sums are not finite.
+template <bool BKN>
+__device__ __forceinline__ void f32_block(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc,
+                                       int M, int N, int K, int m0, int n0) {
+    const int lane = threadIdx.x & 63, r = lane & 31, kh = 8 * (lane >> 5);
+    if (m0 >= M || n0 >= N) return;
+    const float *pa = A + (int64_t)min(m0 + r, M - 1) * lda;
+    const int n = min(n0 + r, N - 1);
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    for (int k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const int k = k0 + kh + s, kc = min(k, K - 1);
+            const float a = pa[kc], b = BKN ? B[(int64_t)kc * ldb + n] : B[(int64_t)n * ldb + kc];
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < K ? a : 0.0f, k < K ? b : 0.0f, acc, 0, 0, 0);
+        }
+    }
+    if (n0 + r >= N) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int row = m0 + acc_row(e, lane);
+        if (row < M) C[(int64_t)row * ldc + n0 + r] = acc[e];
+    }
+}
+
+// Block tile (32 TM WM) x (32 TN WN), WM x WN wavefronts of TM x TN 32 x 32 accumulators, K in
+// chunks of KC through two LDS stages. Every thread loads 16-byte pieces of the operands'
+// rows, splits them into the three parts and stores those as planes of [row][KC] bf16; each
+// operand value is split once per block and read back as 16-byte MFMA operands.
+// What bounds it: at 4096 x 3072 x 3072 the MFMA, 400 us = 1.16 PFLOP/s of bf16 products (the
+// f32 MFMA kernel took 637); with one block per CU the serial latency of a chunk (load, split,
+// LDS round trip, MFMAs), which is why few tiles take deep chunks and 8 wavefronts: 512 x 3072,
+// K = 768 in 64 x 128 tiles 22.9 us with 8 wavefronts and KC = 32, 25.8 with 4, 27.6 at KC =
+// 16. Loads two or three chunks ahead and MFMAs interleaved with the split by hand gained
+// nothing. Batched 512 x 64 x 512 over 384 heads: 168 -> 153 us, its f32 output's stores.
+// VEC: K, pitches and strides multiples of 4, 16-byte aligned operands, and N % 4 == 0 for
+// BKN; otherwise values are loaded one by one.
+template <int TM, int TN, int WM, int WN, int KC, bool BKN, bool VEC>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
     const float *__restrict__ A, int64_t lda, const float *__restrict__ B, int64_t ldb, float *__restrict__ C,
     int64_t ldc, F32Strides s1, F32Strides s2, int M, int N, int K, int tilesN) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NT = 64 * WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
+    constexpr int P = 2 * KC + 16;                // LDS bytes per row of a plane: 16-byte groups of 16 rows in distinct banks
+    constexpr int PLA = BM * P, PLB = BN * P, STAGE = 3 * (PLA + PLB);
+    constexpr int AV = BM * KC / 4 / NT;          // float4 per thread per chunk
+    constexpr int KNI = (KC / 2) * (BN / 4);      // KN: (k pair, 4 columns) items of a chunk
+    constexpr int BV = BKN ? 2 * ((KNI + NT - 1) / NT) : BN * KC / 4 / NT;
+    static_assert(AV >= 1 && BV >= 1 && (KNI % NT == 0 || KNI < NT) && STAGE * 2 <= 128 * 1024, "tile");
+    const bool kn_mine = KNI >= NT || (int)threadIdx.x < KNI;
+    __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
     const int64_t y = blockIdx.y, z = blockIdx.z;
     A += y * s1.a + z * s2.a;
     B += y * s1.b + z * s2.b;
     C += y * s1.c + z * s2.c;
-    const int tm = blockIdx.x / tilesN, tn = blockIdx.x % tilesN;
-    const int m0 = tm * 64 * WM + (wave / WN) * 64, n0 = tn * 64 * WN + (wave % WN) * 64;
-    if (m0 >= M || n0 >= N) return;  // no barriers: a wavefront with no rows or columns just leaves
-    const int r = lane & 31, kh = 8 * (lane >> 5);
+    const int logical = xcd_logical_tile(blockIdx.x, gridDim.x);
+    const int bm0 = (logical / tilesN) * BM, bn0 = (logical % tilesN) * BN;
+    const int wm = wave / WN, wn = wave % WN;
 
-    const float *pa[2], *pb[2];
+    // Loader: KC / 4 consecutive threads per row, 16 bytes each, so rows are read in whole
+    // KC * 4-byte runs. KN: thread items of two k rows x 4 columns, 4 items side by side.
+    constexpr int LPR = KC / 4;
+    const int lk = 4 * (tid % LPR), lr = tid / LPR;
+    const float *ga[AV], *gb[BV];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        pa[t] = A + (int64_t)min(m0 + 32 * t + r, M - 1) * lda;
+    for (int i = 0; i < AV; ++i) ga[i] = A + (int64_t)min(bm0 + lr + (NT / LPR) * i, M - 1) * lda;
+    // KN items: k pair pk, columns 4 pg ..
+    constexpr int NPAIR = KC / 2;
+    const int pk = (tid / 4) % NPAIR;
+    auto pg = [&](int i) { return min(tid % 4 + 4 * ((tid / 4 + (NT / 4) * i) / NPAIR), BN / 4 - 1); };
+#pragma unroll
+    for (int i = 0; i < BV; ++i) {
+        if (BKN) gb[i] = i < BV / 2 ? B + (VEC ? min(bn0 + 4 * pg(i), N - 4) : 0) : nullptr;
+        else gb[i] = B + (int64_t)min(bn0 + lr + (NT / LPR) * i, N - 1) * ldb;
+    }
+    f32x4 ra[AV], rb[BV];
+    auto load_row = [&](const float *p, int k) -> f32x4 {
+        if (VEC) return *reinterpret_cast<const f32x4 *>(p + min(k, K - 4));
+        return f32x4{p[min(k, K - 1)], p[min(k + 1, K - 1)], p[min(k + 2, K - 1)], p[min(k + 3, K - 1)]};
+    };
+    auto load = [&](int c) {
+        const int k = KC * c + lk;
+#pragma unroll
+        for (int i = 0; i < AV; ++i) ra[i] = load_row(ga[i], k);
+        if (BKN) {
+#pragma unroll
+            for (int i = 0; i < BV / 2; ++i)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int64_t kr = (int64_t)min(KC * c + 2 * pk + u, K - 1) * ldb;
+                    if (VEC) rb[2 * i + u] = *reinterpret_cast<const f32x4 *>(gb[i] + kr);
+                    else {
+                        const int n = bn0 + 4 * pg(i);
+                        rb[2 * i + u] = f32x4{B[kr + min(n, N - 1)], B[kr + min(n + 1, N - 1)], B[kr + min(n + 2, N - 1)],
+                                                    B[kr + min(n + 3, N - 1)]};
+                    }
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BV; ++i) rb[i] = load_row(gb[i], k);
+        }
+    };
+    auto put_row = [&](char *plane, int stride, int row, f32x4 v, int k) {
+        // k >= K counts as zero
+        if (VEC) {
+            if (k >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
+        } else {
+            v.x = k < K ? v.x : 0.f, v.y = k + 1 < K ? v.y : 0.f, v.z = k + 2 < K ? v.z : 0.f, v.w = k + 3 < K ? v.w : 0.f;
+        }
+        uint32_t h0, m0, l0, h1, m1, l1;
+        split3_pair(v.x, v.y, h0, m0, l0);
+        split3_pair(v.z, v.w, h1, m1, l1);
+        char *d = plane + row * P + 2 * lk;
+        *reinterpret_cast<uint2 *>(d) = make_uint2(h0, h1);
+        *reinterpret_cast<uint2 *>(d + stride) = make_uint2(m0, m1);
+        *reinterpret_cast<uint2 *>(d + 2 * stride) = make_uint2(l0, l1);
+    };
+    auto store = [&](int c, char *st) {
+#pragma unroll
+        for (int i = 0; i < AV; ++i) put_row(st, PLA, lr + (NT / LPR) * i, ra[i], KC * c + lk);
+        char *bp = st + 3 * PLA;
+        if (BKN) {
+#pragma unroll
+            for (int i = 0; i < BV / 2; ++i) {
+                if (!kn_mine) continue;
+                f32x4 u = rb[2 * i], w = rb[2 * i + 1];
+                const int k = KC * c + 2 * pk;
+                if (k >= K) u = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (k + 1 >= K) w = f32x4{0.f, 0.f, 0.f, 0.f};
+                const float uu[4] = {u.x, u.y, u.z, u.w}, ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    uint32_t h, m, l;
+                    split3_pair(uu[e], ww[e], h, m, l);
+                    char *d = bp + (4 * pg(i) + e) * P + 4 * pk;
+                    *reinterpret_cast<uint32_t *>(d) = h;
+                    *reinterpret_cast<uint32_t *>(d + PLB) = m;
+                    *reinterpret_cast<uint32_t *>(d + 2 * PLB) = l;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BV; ++i) put_row(bp, PLB, lr + (NT / LPR) * i, rb[i], KC * c + lk);
+        }
+    };
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][t][e] = 0.0f;
+    // Chunk c + 1 is split into the other stage while chunk c's MFMAs run, and its registers
+    // take chunk c + 2. Past the last chunk the loads re-read it and the stage is not used: no
+    // branch, so that all of an iteration is scheduled together.
+    const int nc = (K + KC - 1) / KC, last = nc - 1;
+    load(0);
+    store(0, lds);
+    load(min(1, last));
+    lds_barrier();
+    for (int c = 0; c < nc; ++c) {
+        char *cur = lds + (c & 1) * STAGE, *nxt = lds + ((c & 1) ^ 1) * STAGE;
+        bf16x8 pa[KC / 16][TM][3], pb[KC / 16][TN][3];
+#pragma unroll
+        for (int s = 0; s < KC / 16; ++s) {
+            const char *ap = cur + (wm * 32 * TM + r) * P + 32 * s + 16 * hf;
+            const char *bp = cur + 3 * PLA + (wn * 32 * TN + r) * P + 32 * s + 16 * hf;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) pa[s][i][q] = *reinterpret_cast<const bf16x8 *>(ap + q * PLA + 32 * i * P);
+#pragma unroll
+                for (int t = 0; t < TN; ++t) pb[s][t][q] = *reinterpret_cast<const bf16x8 *>(bp + q * PLB + 32 * t * P);
+            }
+        }
+        store(c + 1, nxt);
+        load(min(c + 2, last));
+#pragma unroll
+        for (int s = 0; s < KC / 16; ++s) mfma_parts<TM, TN>(pa[s], pb[s], acc);
+        lds_barrier();
+    }
+    const int m0 = bm0 + 32 * TM * wm, n0 = bn0 + 32 * TN * wn;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc)) != 0, 0)) {
+        for (int u = 0; u < TM * TN; ++u)
+            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            const int col = n0 + 32 * t + r;
+            if (col >= N) continue;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + 32 * i + acc_row(e, lane);
+                if (row < M) C[(int64_t)row * ldc + col] = acc[i][t][e];
+            }
+        }
+}
+
+// K split: 4 wavefronts per (32 TM) x (32 TN) tile, wavefront w taking the 32-deep chunks w, w +
+// 4, ... Each lane loads its own MFMA operands (8 consecutive k of its row per step) and splits
+// them in registers: no LDS and no barrier until the four partial sums are added in a fixed
+// order. Bound by the row-per-lane loads (32 rows per instruction), so it only pays where the
+// tiles are few and K is long: 128 x 768, K = 768 8.4 us against 17.8 in gemm_f32_tile's 64 x
+// 64 tiles (61.5 on the f32 MFMA), 512 x 768 12.0 against 18.1, 512 x 768, K = 3072 36.8
+// against 61.7; but 512 x 3072, K = 768 32.2 against 22.9. VEC as gemm_f32_tile's.
+template <int TM, int TN, bool BKN, bool VEC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restrict__ A, int64_t lda,
+                                                          const float *__restrict__ B, int64_t ldb, float *__restrict__ C,
+                                                          int64_t ldc, F32Strides s1, F32Strides s2, int M, int N, int K,
+                                                          int tilesN) {
+    constexpr int WK = 4, NT = 256, BM = 32 * TM, BN = 32 * TN;
+    constexpr int P = BN + 8;  // LDS row pitch: rows 4 apart start 32 banks apart
+    __shared__ __attribute__((aligned(16))) float red[WK][BM * P];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t y = blockIdx.y, z = blockIdx.z;
+    A += y * s1.a + z * s2.a;
+    B += y * s1.b + z * s2.b;
+    C += y * s1.c + z * s2.c;
+    const int logical = xcd_logical_tile(blockIdx.x, gridDim.x);
+    const int m0 = (logical / tilesN) * BM, n0 = (logical % tilesN) * BN;
+    const int r = lane & 31, hf = lane >> 5;
+
+    const float *pa[TM], *pb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) pa[i] = A + (int64_t)min(m0 + 32 * i + r, M - 1) * lda;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
         const int n = min(n0 + 32 * t + r, N - 1);
         pb[t] = BKN ? B + n : B + (int64_t)n * ldb;
     }
-    auto load = [&](int k0, float (&a)[2][8], float (&b)[2][8]) {
+    float ra[2][TM][8], rb[2][TN][8];
+    auto load_row = [&](const float *p, int k, float (&v)[8]) {
+        if (VEC) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            load8_row<VEC>(pa[t], k0 + kh, K, a[t]);
-            if (BKN) load8_col(pb[t], ldb, k0 + kh, K, b[t]);
-            else load8_row<VEC>(pb[t], k0 + kh, K, b[t]);
-        }
-    };
-
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    // The next K block's loads are issued before the current block's 32 MFMAs (2048
-    // cycles). Loads past K stay in bounds (clamped addresses); KM zeroes their values
-    // before use (the last block is then partial). An explicit two-set ping-pong with
-    // scheduling barriers measured 10-45% slower on MI355X.
-    float a[2][8], b[2][8], na[2][8], nb[2][8];
-    load(0, a, b);
-    for (int k0 = 0; k0 < K; k0 += F32_KB) {
-        load(k0 + F32_KB, na, nb);
-        if (KM) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                kmask(a[t], k0 + kh, K);
-                kmask(b[t], k0 + kh, K);
+            for (int q = 0; q < 2; ++q) {
+                const f32x4 x = *reinterpret_cast<const f32x4 *>(p + min(k + 4 * q, K - 4));
+                v[4 * q] = x.x, v[4 * q + 1] = x.y, v[4 * q + 2] = x.z, v[4 * q + 3] = x.w;
             }
-        }
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                a[t][s] = na[t][s];
-                b[t][s] = nb[t][s];
-            }
-    }
-
-    // accumulator element e of lane l: row 8*(e/4) + 4*(l/32) + e%4, column l%32
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + 32 * j + r;
-            if (col >= N) continue;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = m0 + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                if (row < M) C[(int64_t)row * ldc + col] = acc[i][j][e];
-            }
-        }
-}
-
-// LDS-staged form (the one used whenever the operands allow 16-byte loads: K, pitches
-// and strides multiples of 4, 16-byte aligned bases, and N % 4 == 0 for BKN). The block's
-// (64*WM) x (64*WN) tile takes K in 16-deep chunks through a double LDS buffer: every
-// thread loads whole 16-byte pieces of operand rows (coalesced, 4 lanes per 64-byte row
-// chunk), the next chunk's loads are in flight during the current chunk's 32 MFMAs per
-// wavefront, and one barrier per chunk hands the buffers over. The MFMA operands come
-// from LDS in the same k order as gemm_f32_bt (lane half h takes k = 8h + s), so the two
-// forms give the same bits. A rows and B columns past M / N are clamped on load, k >= K
-// is zeroed when stored to LDS. Measured on MI355X at one config-4 layer's attention
-// (768 problems per launch): QK^T 515 -> 360 us, scores . V 392 -> 280 us.
-template <int WM, int WN, bool BKN>
-__global__ __launch_bounds__(256) void gemm_f32_bt_lds(
-    const float *__restrict__ A, int64_t lda, const float *__restrict__ B, int64_t ldb, float *__restrict__ C,
-    int64_t ldc, F32Strides s1, F32Strides s2, int M, int N, int K, int tilesN) {
-    constexpr int BM = 64 * WM, BN = 64 * WN, BK = F32_KB, KL = BK / 2;
-    constexpr int AP = BK + 4;                        // LDS pitch of a [row][k] tile (floats)
-    constexpr int BP = BN + 4;                        // LDS pitch of a [k][n] tile (floats)
-    constexpr int A_SZ = BM * AP, B_SZ = BKN ? BK * BP : BN * AP;
-    constexpr int AV = BM * (BK / 4) / 256;           // float4 per thread for A
-    constexpr int BV = (BKN ? BK * (BN / 4) : BN * (BK / 4)) / 256;
-    static_assert(AV >= 1 && BV >= 1, "tile too small");
-    __shared__ __attribute__((aligned(16))) float lds[2][A_SZ + B_SZ];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t y = blockIdx.y, z = blockIdx.z;
-    A += y * s1.a + z * s2.a;
-    B += y * s1.b + z * s2.b;
-    C += y * s1.c + z * s2.c;
-    const int tm = blockIdx.x / tilesN, tn = blockIdx.x % tilesN;
-    const int bm0 = tm * BM, bn0 = tn * BN;
-    const int wm0 = (wave / WN) * 64, wn0 = (wave % WN) * 64;  // wave tile within the block
-
-    // global source of each staged float4 (k offset added per chunk)
-    const float *ga[AV];
-    int ak[AV], arow_l[AV];
-#pragma unroll
-    for (int i = 0; i < AV; ++i) {
-        const int idx = tid + 256 * i, row = idx / (BK / 4), c4 = idx % (BK / 4);
-        ga[i] = A + (int64_t)min(bm0 + row, M - 1) * lda;
-        ak[i] = 4 * c4;
-        arow_l[i] = row;
-    }
-    const float *gb[BV];
-    int bk_[BV], brow_l[BV];
-#pragma unroll
-    for (int i = 0; i < BV; ++i) {
-        const int idx = tid + 256 * i;
-        if (BKN) {
-            const int kr = idx / (BN / 4), c4 = idx % (BN / 4);
-            gb[i] = B + min(bn0 + 4 * c4, N - 4);  // + k*ldb per element row
-            bk_[i] = kr;
-            brow_l[i] = 4 * c4;
         } else {
-            const int row = idx / (BK / 4), c4 = idx % (BK / 4);
-            gb[i] = B + (int64_t)min(bn0 + row, N - 1) * ldb;
-            bk_[i] = 4 * c4;
-            brow_l[i] = row;
-        }
-    }
-    f32x4 ra[AV], rb[BV];
-    auto gload = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < AV; ++i) ra[i] = *reinterpret_cast<const f32x4 *>(ga[i] + min(k0 + ak[i], K - 4));
-#pragma unroll
-        for (int i = 0; i < BV; ++i) {
-            if (BKN) rb[i] = *reinterpret_cast<const f32x4 *>(gb[i] + (int64_t)min(k0 + bk_[i], K - 1) * ldb);
-            else rb[i] = *reinterpret_cast<const f32x4 *>(gb[i] + min(k0 + bk_[i], K - 4));
+            for (int e = 0; e < 8; ++e) v[e] = p[min(k + e, K - 1)];
         }
     };
-    auto lstore = [&](int k0, float *buf) {
+    auto load = [&](int j, int c) {  // step j of chunk c
+        const int k = 32 * c + 16 * j + 8 * hf;
 #pragma unroll
-        for (int i = 0; i < AV; ++i) {
-            f32x4 v = ra[i];
-            if (k0 + ak[i] >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
-            *reinterpret_cast<f32x4 *>(buf + arow_l[i] * AP + ak[i]) = v;
-        }
+        for (int i = 0; i < TM; ++i) load_row(pa[i], k, ra[j][i]);
 #pragma unroll
-        for (int i = 0; i < BV; ++i) {
-            f32x4 v = rb[i];
+        for (int t = 0; t < TN; ++t) {
             if (BKN) {
-                if (k0 + bk_[i] >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
-                *reinterpret_cast<f32x4 *>(buf + A_SZ + bk_[i] * BP + brow_l[i]) = v;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rb[j][t][e] = pb[t][(int64_t)min(k + e, K - 1) * ldb];
             } else {
-                if (k0 + bk_[i] >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
-                *reinterpret_cast<f32x4 *>(buf + A_SZ + brow_l[i] * AP + bk_[i]) = v;
+                load_row(pb[t], k, rb[j][t]);
             }
         }
     };
-
-    f32x16 acc[2][2];
+    auto split8 = [&](const float (&x)[8], bf16x8 (&p)[3]) {
+        uint32_t h[4], m[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 4; ++i) split3_pair(x[2 * i], x[2 * i + 1], h[i], m[i], l[i]);
+        p[0] = __builtin_bit_cast(bf16x8, (u32x4{h[0], h[1], h[2], h[3]}));
+        p[1] = __builtin_bit_cast(bf16x8, (u32x4{m[0], m[1], m[2], m[3]}));
+        p[2] = __builtin_bit_cast(bf16x8, (u32x4{l[0], l[1], l[2], l[3]}));
+    };
+    f32x16 acc[TM][TN];
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    const int r = lane & 31, h = lane >> 5;
-    // lane half h takes k = KL*h + s of the chunk in MFMA step s (the same for A and B)
-    auto compute = [&](const float *buf) {
-        float a[2][KL], b[2][KL];
+        for (int t = 0; t < TN; ++t)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const float *pa = buf + (wm0 + 32 * t + r) * AP + KL * h;
+            for (int e = 0; e < 16; ++e) acc[i][t][e] = 0.0f;
+    const int nc = (K + 31) / 32;
+    if (wave < nc) {  // uniform
+        load(0, wave);
+        load(1, wave);
+        for (int c = wave; c < nc; c += WK) {
+            const bool more = c + WK < nc;
 #pragma unroll
-            for (int q = 0; q < KL / 4; ++q) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(pa + 4 * q);
-                a[t][4 * q] = v.x; a[t][4 * q + 1] = v.y; a[t][4 * q + 2] = v.z; a[t][4 * q + 3] = v.w;
-            }
-            if (BKN) {
-                const float *pb = buf + A_SZ + (KL * h) * BP + wn0 + 32 * t + r;
+            for (int j = 0; j < 2; ++j) {
+                if (32 * c + 32 > K) {  // the last chunk: k past K counts as zero in both operands
+                    const int k = 32 * c + 16 * j + 8 * hf;
 #pragma unroll
-                for (int s = 0; s < KL; ++s) b[t][s] = pb[s * BP];
-            } else {
-                const float *pb = buf + A_SZ + (wn0 + 32 * t + r) * AP + KL * h;
+                    for (int e = 0; e < 8; ++e) {
 #pragma unroll
-                for (int q = 0; q < KL / 4; ++q) {
-                    const f32x4 v = *reinterpret_cast<const f32x4 *>(pb + 4 * q);
-                    b[t][4 * q] = v.x; b[t][4 * q + 1] = v.y; b[t][4 * q + 2] = v.z; b[t][4 * q + 3] = v.w;
+                        for (int i = 0; i < TM; ++i) ra[j][i][e] = k + e < K ? ra[j][i][e] : 0.0f;
+#pragma unroll
+                        for (int t = 0; t < TN; ++t) rb[j][t][e] = k + e < K ? rb[j][t][e] : 0.0f;
+                    }
                 }
+                bf16x8 qa[TM][3], qb[TN][3];
+#pragma unroll
+                for (int i = 0; i < TM; ++i) split8(ra[j][i], qa[i]);
+#pragma unroll
+                for (int t = 0; t < TN; ++t) split8(rb[j][t], qb[t]);
+                if (more) load(j, c + WK);
+                mfma_parts<TM, TN>(qa, qb, acc);
             }
         }
-#pragma unroll
-        for (int s = 0; s < KL; ++s)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
-    };
-
-    const int nc = (K + BK - 1) / BK;
-    gload(0);
-    lstore(0, lds[0]);
-    __syncthreads();
-    // The next chunk's loads are unconditional (past K the clamped addresses stay in the
-    // operands and lstore zeroes the values), so the compiler's wait counts stay exact.
-    for (int c = 0; c < nc; ++c) {
-        gload((c + 1) * BK);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(lds[c & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        lstore((c + 1) * BK, lds[(c + 1) & 1]);
-        __syncthreads();
     }
-
-    const bool live = bm0 + wm0 < M && bn0 + wn0 < N;
-    if (!live) return;
+    if (__builtin_expect(__syncthreads_or(any_nonfinite<TM, TN>(acc)), 0)) {
+        for (int u = wave; u < TM * TN; u += WK)
+            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+        return;
+    }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = bn0 + wn0 + 32 * j + r;
-            if (col >= N) continue;
+        for (int t = 0; t < TN; ++t)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = bm0 + wm0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (row < M) C[(int64_t)row * ldc + col] = acc[i][j][e];
-            }
+            for (int e = 0; e < 16; ++e) red[wave][(32 * i + acc_row(e, lane)) * P + 32 * t + r] = acc[i][t][e];
+    __syncthreads();
+    constexpr int RL = BN / 4, RP = NT / RL, NG = BM * RL / NT;  // 16-byte groups per row; rows per pass; passes
+    static_assert(BM * RL % NT == 0, "whole passes");
+    const int c4 = 4 * (tid % RL), r0 = tid / RL, col = n0 + c4;
+    const bool vst = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C & 15) == 0;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int at = (r0 + RP * g) * P + c4, row = m0 + r0 + RP * g;
+        f32x4 v = *reinterpret_cast<const f32x4 *>(&red[0][at]);
+#pragma unroll
+        for (int w = 1; w < WK; ++w) {
+            const f32x4 o = *reinterpret_cast<const f32x4 *>(&red[w][at]);
+            v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
         }
+        if (row >= M) continue;
+        float *o = C + (int64_t)row * ldc + col;
+        if (vst) {
+            if (col < N) *reinterpret_cast<f32x4 *>(o) = v;
+        } else {
+            const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (col + u < N) o[u] = x[u];
+        }
+    }
 }
-
 
 // C = 0 for a K = 0 product (the empty dot product), grid (ceil(M*N/256), inner, outer).
 __global__ __launch_bounds__(256) void fill_zero_f32(float *__restrict__ C, int64_t ldc, int64_t sc1, int64_t sc2,

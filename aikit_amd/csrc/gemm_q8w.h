@@ -46,7 +46,6 @@
 
 namespace enchip {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Bytes of one A stage in LDS: BM / 32 row blocks x 3 parts x 2 steps x 1 KiB.
 __host__ __device__ constexpr int q8w_stage_bytes(int bm) { return (bm / 32) * 6 * 1024; }

@@ -576,11 +576,12 @@ def other_configs(ctx, torch, stream, ceilings):
             att[f"{tag}_frac_bf16_mfma_peak"] = 3 * 2 * flops / t / PEAK_BF16_FLOPS
     ctx.set_attention_products(enchip.ATT_DEFAULT)
     att.update({"S": S, "L": L, "heads": H, "head_dim": hd, "gflop_per_product": flops / 1e9,
-                "kernels": "enchip::gemm_f32_bt_lds<2, 2, false> (QK^T), enchip::gemm_f32_bt_lds<4, 1, true> (PV), "
+                "kernels": "enchip::gemm_f32_tile<2, 2, 2, 2, 16, false, true> (QK^T), "
+                           "enchip::gemm_f32_tile<1, 2, 4, 1, 16, true, true> (PV), "
                            "enchip::attention_f32<64> (fused, f32 MFMA), enchip::attention_split_bf16<64, true> "
                            "(fused, split-bf16 MFMA), enchip::attention_flash<64, 8, true, false|true> (fused online softmax, "
                            "bfloat16 / half split products; the half split is the default)",
-                "note": "one config-4 layer's attention products (qk, pv: f32 MatmulBT on v_mfma_f32_32x32x2_f32), all "
+                "note": "one config-4 layer's attention products (qk, pv: f32 MatmulBT, six bf16 products of split operands), all "
                         "768 (sequence, head) problems per launch, operands resident; bytes = operands read once + "
                         "output written once; softmax not included in qk/pv, included in the fused forms"})
     out["attention_f32_cfg4_layer"] = att

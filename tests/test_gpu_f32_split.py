@@ -1,0 +1,91 @@
+"""GPU tests of the f32 MatmulBT's split products (three bf16 parts per operand, six products):
+every tile form at its edges against float64 with the bound its roundings give, operands the
+split cannot hold, and one result per problem whatever the batch and layout."""
+import numpy as np
+import pytest
+
+from aikit_amd import enchip, workloads
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): the K split in 32 x 32, 64 x 32 and 64 x 64 tiles; 64 x 64, 64 x 128, 128 x 64
+# and 128 x 128 tiles; with remainders in every dimension, K below and past a chunk, and
+# K or N not a multiple of 4 (values loaded one by one)
+SHAPES = [(33, 300, 132, "k32"), (500, 257, 1000, "k64x32"), (1, 1024, 4097, "k"), (70, 40, 100, "64"), (65, 33, 65, "64"),
+          (500, 200, 2050, "64x128"), (3000, 100, 60, "128x64"), (1200, 96, 1500, "128x64"), (2100, 52, 2052, "128"),
+          (1999, 31, 2301, "128"), (2, 5, 3, "64")]
+
+
+def bound(a, b, K):
+    """|C - exact| <= (adds + 2) 2^-24 sum |a b|: 6 rounded adds of the running sum per 16-deep
+    step, the K split's 3 and the products left out (under 2^-25 each)."""
+    return (6 * -(-K // 16) + 3 + 2) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T)
+
+
+@pytest.mark.parametrize("M,K,N,form", SHAPES)
+@pytest.mark.parametrize("layout", [enchip.B_NK, enchip.B_KN])
+def test_split_products_within_their_rounding_bound(ctx, M, K, N, form, layout):
+    import torch
+
+    g = workloads.rng(5000 + M + K + N)
+    a = g.standard_normal((M, K)).astype(np.float32)
+    b = g.standard_normal((N, K)).astype(np.float32)
+    a *= np.exp2(g.integers(-8, 9, size=(M, K))).astype(np.float32)  # a spread of magnitudes
+    print(f"[case] f32 split M={M} K={K} N={N} layout={layout} ({form})", flush=True)
+    da = torch.from_numpy(a).cuda()
+    db = torch.from_numpy(np.ascontiguousarray(b if layout == enchip.B_NK else b.T)).cuda()
+    dc = torch.full((M, N), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.matmul_bt_f32_dev(da.data_ptr(), K, db.data_ptr(), K if layout == enchip.B_NK else N, layout, dc.data_ptr(), N,
+                          M, K, N)
+    torch.cuda.synchronize()
+    ref = a.astype(np.float64) @ b.astype(np.float64).T
+    assert np.all(np.abs(dc.cpu().numpy() - ref) <= bound(a, b, K))
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 300, 200), (80, 64, 70), (2100, 64, 2052)])
+def test_infinities_nans_and_the_largest_floats(ctx, M, K, N):
+    # What f32 arithmetic gives: an infinity times a nonzero value is an infinity, times zero
+    # NaN; a float that rounds to infinity in bf16 stays finite; the other rows are untouched.
+    g = workloads.rng(77 + M)
+    a = g.standard_normal((M, K)).astype(np.float32)
+    b = np.abs(g.standard_normal((N, K))).astype(np.float32) + np.float32(0.5)
+    a[3, 5] = np.inf
+    a[7, K - 1] = -np.inf
+    a[11, 2] = np.nan
+    a[M - 1] = 0
+    a[M - 1, 1] = np.float32(3.4028235e38)  # the largest float, times 0.5 .. : finite or inf as f32 has it
+    b[4, 5] = 0  # inf * 0
+    b[N - 1, 1] = np.float32(0.25)
+    with np.errstate(all="ignore"):
+        want = (a.astype(np.float64)[:, None, :] * b.astype(np.float64)[None, :, :]).sum(-1) if M < 1000 else None
+        got = ctx.matmul_bt_f32(a, b)
+        assert np.all(np.isposinf(np.delete(got[3], 4))) and np.isnan(got[3, 4])
+        assert np.all(np.isneginf(got[7])) and np.all(np.isnan(got[11]))
+        big = np.float32(3.4028235e38) * b[:, 1]  # one product: its f32 rounding, infinities included
+        assert np.array_equal(got[M - 1], big)
+        rows = np.setdiff1d(np.arange(M), [3, 7, 11, M - 1])
+        if want is not None:
+            # blocks that hold a special value run on the f32 MFMA: at most one rounded add per product
+            f32 = (K + 2) * 2.0**-24 * (np.abs(a[rows]).astype(np.float64) @ np.abs(b).astype(np.float64).T)
+            assert np.all(np.abs(got[rows] - want[rows]) <= f32)
+        assert np.isfinite(got[rows]).all()
+
+
+def test_a_batch_gives_each_problem_its_own_bits(ctx):
+    # 40 problems of one shape in a launch (larger tiles than one alone would get) and one by one
+    import torch
+
+    g = workloads.rng(9)
+    for M, K, N in ((96, 512, 160), (130, 300, 64), (64, 64, 128)):
+        a = torch.from_numpy(g.standard_normal((40, M, K)).astype(np.float32)).cuda()
+        b = torch.from_numpy(g.standard_normal((40, N, K)).astype(np.float32)).cuda()
+        c1, c2 = torch.empty((40, M, N), device="cuda"), torch.empty((40, M, N), device="cuda")
+        torch.cuda.synchronize()
+        print(f"[case] batch of 40 M={M} K={K} N={N}", flush=True)
+        ctx.matmul_bt_f32_dev(a.data_ptr(), K, b.data_ptr(), K, enchip.B_NK, c1.data_ptr(), N, M, K, N,
+                              inner=(40, M * K, N * K, M * N))
+        for i in range(40):
+            ctx.matmul_bt_f32_dev(a[i].data_ptr(), K, b[i].data_ptr(), K, enchip.B_NK, c2[i].data_ptr(), N, M, K, N)
+        torch.cuda.synchronize()
+        assert torch.equal(c1.view(torch.int32), c2.view(torch.int32))
