@@ -1616,46 +1616,44 @@ int launch_matmul_q8w(enchip_ctx *c, const Weight &w, const float *A, int64_t ld
         return check_launch(c, "fill_zero_f32");
     }
     const bool vec = w.K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0;
-    // 128 x 256 tiles when they give every CU two workgroups, else 128 x 128 when those
-    // do, else 64 x 64 when those give every CU one; below that the K-split small form
-    // (32 x 64 tiles, or 32 x 32 when 32 x 64 would leave CUs idle). Measured on MI355X:
-    // M = 512, K = 768, N = 2304 takes 24 us as 288 64 x 64 tiles against 31 in the small
-    // form, which re-splits A for each column tile; M = 128, K = 768, N = 768, 24 such
-    // tiles, takes 18 us against 9.
-    const int64_t cus = c->num_cus, cus2 = 2 * cus;
+    // The K-split small form while there is at most one of its 32 x 32 tiles per CU: M = 64, K
+    // = 768, N = 3072 (192 tiles) takes 9.3 us against 11.1 in 32 x 128 tiles, M = 128, N =
+    // 2304 (288) 12.0 against 11.2. 128 x 256 tiles when they fill the CUs: about one each, or
+    // from one and a half (in between, the second round is mostly empty): M = 2048, K = 1024,
+    // N = 4096 (256 tiles) 54 us against 65 in 32 x 128, M = 4096, K = 768, N = 2304 (288) 63
+    // against 56, N = 3072 (384) 66 against 72. Otherwise 32 x 128, K in chunks of 128 while
+    // each CU has one (M = 512, K = 3072, N = 768 29.6 us against 31.8 with 64), else of 64.
+    const int64_t cus = c->num_cus;
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((w.N + bn - 1) / bn); };
-    const int form = tiles(128, 256) >= cus2 ? 2 : tiles(128, 128) >= cus2 ? 1 : tiles(64, 64) >= cus ? 0
-                     : tiles(32, 64) >= cus ? -2 : -1;
-    const bool wide = form > 0;
-    const int bm = form < 0 ? 32 : wide ? 128 : 64, bn = form == 2 ? 256 : form == -2 ? 64 : form == -1 ? 32 : bm;
+    const int64_t big = tiles(128, 256);
+    const int form = tiles(32, 32) <= cus                                            ? 0
+                     : 4 * big >= 3 * cus && (big <= cus || 2 * big >= 3 * cus) ? 3
+                     : tiles(32, 128) <= cus                                         ? 1
+                                                                                     : 2;
+    const int bm = form == 3 ? 128 : 32, bn = form == 3 ? 256 : form == 0 ? 32 : 128;
     const int tilesN = (int)((w.N + bn - 1) / bn);
     // every wavefront reads whole 32-channel blocks of the image up to tilesN * bn
     if ((int64_t)tilesN * bn > w.Np) return fail(c, ENCHIP_ERR_ARG, "gemm_q8w: %d tiles exceed the image", tilesN);
-    // rows per launch: at most 2^30 / tilesN tiles of rows, so the tile index stays an int
-    const int64_t rows = std::max<int64_t>(bm, (((int64_t)1 << 30) / tilesN) / bm * bm);
+    // rows per launch: at most 2^29 / tilesN, so a launch's threads stay below 2^32 (many rows
+    // run in the 128-row form)
+    const int64_t rows = std::max<int64_t>(bm, (((int64_t)1 << 29) / tilesN) / bm * bm);
     for (int64_t r0 = 0; r0 < M; r0 += rows) {
         const int64_t n = std::min(rows, M - r0);
-        const dim3 grid((unsigned)(((n + bm - 1) / bm) * tilesN)), block(256);
+        const dim3 grid((unsigned)(((n + bm - 1) / bm) * tilesN));
         const float *a = A + r0 * lda;
         float *cz = C + r0 * ldc;
-#define Q8W_CALL(TM, TN, VEC)                                                                                   \
-    hipLaunchKernelGGL((gemm_q8w<TM, TN, VEC>), grid, block, 0, s, a, lda, w.d_w, w.d_s, cz, ldc, (int)n,       \
-                       (int)w.N, (int)w.K, (int)w.Kp, tilesN)
-#define Q8W_SMALL(TN, VEC)                                                                                      \
-    hipLaunchKernelGGL((gemm_q8w_small<TN, VEC>), grid, block, 0, s, a, lda, w.d_w, w.d_s, cz, ldc, (int)n,     \
-                       (int)w.N, (int)w.K, (int)w.Kp, tilesN)
-        if (form == -2 && vec) Q8W_SMALL(2, true);
-        else if (form == -2) Q8W_SMALL(2, false);
-        else if (form == -1 && vec) Q8W_SMALL(1, true);
-        else if (form == -1) Q8W_SMALL(1, false);
-        else if (form == 2 && vec) Q8W_CALL(2, 4, true);
-        else if (form == 2) Q8W_CALL(2, 4, false);
-        else if (wide && vec) Q8W_CALL(2, 2, true);
-        else if (wide) Q8W_CALL(2, 2, false);
-        else if (vec) Q8W_CALL(1, 1, true);
-        else Q8W_CALL(1, 1, false);
+#define Q8W_CALL(KERNEL, THREADS)                                                                                  \
+    hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, s, a, lda, w.d_w, w.d_s, cz, ldc, (int)n, (int)w.N, (int)w.K, \
+                       (int)w.Kp, tilesN)
+        if (form == 0 && vec) Q8W_CALL(gemm_q8w_small<true>, 256);
+        else if (form == 0) Q8W_CALL(gemm_q8w_small<false>, 256);
+        else if (form == 1 && vec) Q8W_CALL((gemm_q8w<1, 1, 1, 4, 128, 4, true>), 256);
+        else if (form == 1) Q8W_CALL((gemm_q8w<1, 1, 1, 4, 128, 4, false>), 256);
+        else if (form == 2 && vec) Q8W_CALL((gemm_q8w<1, 1, 1, 4, 64, 4, true>), 256);
+        else if (form == 2) Q8W_CALL((gemm_q8w<1, 1, 1, 4, 64, 4, false>), 256);
+        else if (vec) Q8W_CALL((gemm_q8w<2, 2, 2, 4, 32, 1, true>), 512);
+        else Q8W_CALL((gemm_q8w<2, 2, 2, 4, 32, 1, false>), 512);
 #undef Q8W_CALL
-#undef Q8W_SMALL
     }
     return check_launch(c, "gemm_q8w");
 }

@@ -22,17 +22,9 @@
 // read straight into registers, 16 bytes per lane per block. The MFMA's lane half h
 // supplies depth 8h .. 8h + 7 of each 16-deep step, so step j of a 32-deep chunk takes
 // bytes 8j .. 8j + 7 of the lane's 16, i.e. k = 16h + 8j + (0..7): the A operand is fed in
-// the same k order, so the permutation cancels in the sum. A is row-major f32; each
-// workgroup loads a BM x 32 chunk once, splits it and stores the three bf16 planes in LDS
-// as MFMA operand fragments ((row block, part, step) -> 64 lanes x 16 bytes, lane-contiguous
-// so every ds_read_b128 is free of bank conflicts), double-buffered with one barrier per
-// chunk; the next chunk's A and weight loads are in flight during the current chunk's
-// MFMAs.
-//
-// Tiles. 4 wavefronts in 2 x 2, each (32 TM) x (32 TN) of 32 x 32 accumulators: BM = 64 TM,
-// BN = 64 TN. Rows past M re-read row M - 1 and are not stored; k past K is zero in A (the
-// weight image is zero there too); channels past N read the image's zero padding and are
-// not stored.
+// the same k order, so the permutation cancels in the sum. A is row-major f32. Rows past M
+// re-read row M - 1 and are not stored; k past K is zero in A (the weight image is zero there
+// too); channels past N read the image's zero padding and are not stored.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -45,10 +37,6 @@
 #pragma clang fp contract(off)
 
 namespace enchip {
-
-
-// Bytes of one A stage in LDS: BM / 32 row blocks x 3 parts x 2 steps x 1 KiB.
-__host__ __device__ constexpr int q8w_stage_bytes(int bm) { return (bm / 32) * 6 * 1024; }
 
 // The exact split a = b1 + b2 + b3 of one f32 into the upper halves of t1, t2, t3 (the
 // bf16 bit patterns are t >> 16).
@@ -74,157 +62,163 @@ __device__ __forceinline__ void q8w_widen4(uint32_t w, uint32_t &lo, uint32_t &h
     hi = q8w_pack(__float_as_uint(f2), __float_as_uint(f3));
 }
 
-// Grid: tilesM * tilesN workgroups of 256 threads (XCD-aware order), static LDS of two A
-// stages. W: the fragment-major image of an Np x Kp weight (Kp a multiple of 64, Np of
-// BN); ws[N]. VEC: lda % 4 == 0, K % 4 == 0 and A 16-byte aligned (16-byte loads).
-template <int TM, int TN, bool VEC>
-__global__ __launch_bounds__(256, 2) void gemm_q8w(const float *__restrict__ A, int64_t lda,
-                                                   const int8_t *__restrict__ W, const float *__restrict__ ws,
-                                                   float *__restrict__ C, int64_t ldc, int M, int N, int K, int Kp,
-                                                   int tilesN) {
-    constexpr int BM = 64 * TM;
-    constexpr int STAGE = q8w_stage_bytes(BM);
-    constexpr int EPT = BM / 8;        // A elements per thread per chunk: 8 or 16 consecutive k
-    constexpr int TPR = 32 / EPT;      // threads per row
+// Grid: tilesM * tilesN workgroups (XCD-aware order). Block tile (32 TM WM) x (32 TN WN), WM x
+// WN wavefronts of TM x TN 32 x 32 accumulators, K in chunks of KC: every thread loads 16-byte
+// pieces of A's rows, splits them and stores the three parts as planes of [row][KC] bf16 (rows
+// 16 bytes apart from a multiple of 128, so 32 rows' 16-byte operand reads fall in distinct
+// banks), double-buffered. The 16-deep steps rotate over NACC sets of accumulators, added in
+// order at the end: shorter sums, and MFMAs that do not wait for the one before.
+// W: the fragment-major image of an Np x Kp weight (Kp a multiple of 64, Np of BN); ws[N].
+// VEC: lda % 4 == 0, K % 4 == 0 and A 16-byte aligned (16-byte loads).
+// What bounds it: with a block or two per CU the serial latency of a chunk, hence 32-row tiles
+// and deep chunks; with many tiles the MFMA and the splitting's VALU work. Measured on MI355X
+// against the form before (64 x 64 to 128 x 256 tiles, 32-deep chunks, branches around the
+// next chunk's loads), us: 512 x 2304, K = 768 23.2 -> 14.6, 1024 x 768 21.1 -> 11.2, 2048 x
+// 768, K = 3072 74.1 -> 44.3, all in 32 x 128 tiles; 32768 x 3072, K = 768 475 -> 440 (1.05
+// PFLOP/s of bf16 products) and 32768 x 768, K = 3072 465 -> 404 in 128 x 256. Error against
+// float64 at K = 768: 1.4e-7 with NACC = 4, 2.6e-7 with 1 (2.6e-7 before). 256 x 256 tiles
+// with 8 or 16 wavefronts were no faster.
+template <int TM, int TN, int WM, int WN, int KC, int NACC, bool VEC>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_q8w(
+    const float *__restrict__ A, int64_t lda, const int8_t *__restrict__ W, const float *__restrict__ ws,
+    float *__restrict__ C, int64_t ldc, int M, int N, int K, int Kp, int tilesN) {
+    constexpr int NT = 64 * WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, KB = KC / 32;
+    constexpr int P = 2 * KC + 16, PL = BM * P, STAGE = 3 * PL;
+    constexpr int LPR = KC / 4, AV = BM * LPR / NT;
+    static_assert(AV >= 1 && BM * LPR % NT == 0, "tile");
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
     const int logical = xcd_logical_tile(blockIdx.x, gridDim.x);
-    const int m0 = (logical / tilesN) * BM, n0 = (logical % tilesN) * (64 * TN);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int nk = Kp / 32;
-
-    // ---- A loader: row lrow of the tile, k koff .. koff + EPT - 1 of each chunk
-    const int lrow = tid / TPR, koff = EPT * (tid % TPR);
-    const float *arow = A + (int64_t)min(m0 + lrow, M - 1) * lda;
-    float av[EPT];
-    auto load_a = [&](int kc) {
-        const int k0 = 32 * kc + koff;
-        if (32 * kc + 32 <= K) {  // uniform: the whole chunk is inside the row
-            if (VEC) {
+    const int m0 = (logical / tilesN) * BM, n0 = (logical % tilesN) * BN;
+    const int wm = wave / WN, wn = wave % WN;
+    const int lk = 4 * (tid % LPR), lr = tid / LPR;
+    const float *ga[AV];
 #pragma unroll
-                for (int i = 0; i < EPT / 4; ++i) {
-                    const f32x4 t = *reinterpret_cast<const f32x4 *>(arow + k0 + 4 * i);
-                    av[4 * i] = t.x;
-                    av[4 * i + 1] = t.y;
-                    av[4 * i + 2] = t.z;
-                    av[4 * i + 3] = t.w;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < EPT; ++i) av[i] = arow[k0 + i];
-            }
-        } else {
-            // the last partial chunk (or past K): clamped reads, zero past K
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) {
-                const float x = arow[min(k0 + i, K - 1)];
-                av[i] = k0 + i < K ? x : 0.0f;
-            }
-        }
-    };
-    // split into the stage's three planes: 8-element groups at k8 = koff + 8g go to lane
-    // (lrow % 32) + 32 (k8 / 16), step (k8 / 8) % 2 of row block lrow / 32
-    auto store_a = [&](int s) {
-        char *base = lds + s * STAGE + (lrow >> 5) * 6144;
-#pragma unroll
-        for (int g = 0; g < EPT / 8; ++g) {
-            const int k8 = koff + 8 * g, ln = (lrow & 31) + 32 * (k8 >> 4), j = (k8 >> 3) & 1;
-            uint32_t t1[8], t2[8], t3[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) q8w_split3(av[8 * g + e], t1[e], t2[e], t3[e]);
-            const u32x4 w1 = {q8w_pack(t1[0], t1[1]), q8w_pack(t1[2], t1[3]), q8w_pack(t1[4], t1[5]),
-                              q8w_pack(t1[6], t1[7])};
-            const u32x4 w2 = {q8w_pack(t2[0], t2[1]), q8w_pack(t2[2], t2[3]), q8w_pack(t2[4], t2[5]),
-                              q8w_pack(t2[6], t2[7])};
-            const u32x4 w3 = {q8w_pack(t3[0], t3[1]), q8w_pack(t3[2], t3[3]), q8w_pack(t3[4], t3[5]),
-                              q8w_pack(t3[6], t3[7])};
-            *reinterpret_cast<u32x4 *>(base + (0 * 2 + j) * 1024 + ln * 16) = w1;
-            *reinterpret_cast<u32x4 *>(base + (1 * 2 + j) * 1024 + ln * 16) = w2;
-            *reinterpret_cast<u32x4 *>(base + (2 * 2 + j) * 1024 + ln * 16) = w3;
-        }
-    };
-
-    // ---- weight fragments: this wave's TN channel blocks, 16 bytes per lane per chunk
+    for (int i = 0; i < AV; ++i) ga[i] = A + (int64_t)min(m0 + lr + (NT / LPR) * i, M - 1) * lda;
+    const int nk32 = Kp / 32;
     const int8_t *wb[TN];
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-        wb[t] = W + ((int64_t)((n0 >> 5) + TN * wn + t) * nk) * 1024 + lane * 16;
-    u32x4 wr[TN];
-    auto load_w = [&](int kc) {
+    for (int t = 0; t < TN; ++t) wb[t] = W + ((int64_t)((n0 >> 5) + TN * wn + t) * nk32) * 1024 + lane * 16;
+    f32x4 ra[AV];
+    u32x4 wr[KB][TN];
+    auto load_a = [&](int c) {
+        const int k = KC * c + lk;
 #pragma unroll
-        for (int t = 0; t < TN; ++t) wr[t] = *reinterpret_cast<const u32x4 *>(wb[t] + (int64_t)kc * 1024);
+        for (int i = 0; i < AV; ++i) {
+            if (VEC) ra[i] = *reinterpret_cast<const f32x4 *>(ga[i] + min(k, K - 4));
+            else
+                ra[i] = f32x4{ga[i][min(k, K - 1)], ga[i][min(k + 1, K - 1)], ga[i][min(k + 2, K - 1)],
+                              ga[i][min(k + 3, K - 1)]};
+        }
     };
-
-    f32x16 acc[TM][TN];
+    auto load_w = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int b = 0; b < KB; ++b)
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
+            for (int t = 0; t < TN; ++t)
+                wr[b][t] = *reinterpret_cast<const u32x4 *>(wb[t] + (int64_t)min(KB * c + b, nk32 - 1) * 1024);
+    };
+    auto store_a = [&](int c, char *st) {
+        const int k = KC * c + lk;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][t][e] = 0.0f;
-
+        for (int i = 0; i < AV; ++i) {
+            f32x4 v = ra[i];  // k past K counts as zero
+            if (VEC) {
+                if (k >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
+            } else {
+                v.x = k < K ? v.x : 0.f, v.y = k + 1 < K ? v.y : 0.f, v.z = k + 2 < K ? v.z : 0.f, v.w = k + 3 < K ? v.w : 0.f;
+            }
+            uint32_t a1[4], a2[4], a3[4];
+            q8w_split3(v.x, a1[0], a2[0], a3[0]);
+            q8w_split3(v.y, a1[1], a2[1], a3[1]);
+            q8w_split3(v.z, a1[2], a2[2], a3[2]);
+            q8w_split3(v.w, a1[3], a2[3], a3[3]);
+            char *d = st + (lr + (NT / LPR) * i) * P + 2 * lk;
+            *reinterpret_cast<uint2 *>(d) = make_uint2(q8w_pack(a1[0], a1[1]), q8w_pack(a1[2], a1[3]));
+            *reinterpret_cast<uint2 *>(d + PL) = make_uint2(q8w_pack(a2[0], a2[1]), q8w_pack(a2[2], a2[3]));
+            *reinterpret_cast<uint2 *>(d + 2 * PL) = make_uint2(q8w_pack(a3[0], a3[1]), q8w_pack(a3[2], a3[3]));
+        }
+    };
+    f32x16 acc[NACC][TM][TN];
+#pragma unroll
+    for (int a = 0; a < NACC; ++a)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[a][i][t][e] = 0.0f;
+    // Chunk c + 1 is split into the other stage while chunk c's MFMAs run, and its registers
+    // take chunk c + 2. Past the last chunk the loads re-read it and the stage is not used: no
+    // branch, so that all of an iteration is scheduled together.
+    const int nc = (Kp + KC - 1) / KC, last = nc - 1;
     load_a(0);
     load_w(0);
-    store_a(0);
+    store_a(0, lds);
+    load_a(min(1, last));
     lds_barrier();
-    for (int kc = 0; kc < nk; ++kc) {
-        // widen this chunk's weight codes, then put the next chunk's loads in flight
-        bf16x8 wq[TN][2];
+    for (int c = 0; c < nc; ++c) {
+        const char *cur = lds + (c & 1) * STAGE;
+        char *nxt = lds + ((c & 1) ^ 1) * STAGE;
 #pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            const uint32_t d[4] = {wr[t].x, wr[t].y, wr[t].z, wr[t].w};
+        for (int b = 0; b < KB; ++b) {
+            bf16x8 wq[TN][2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                uint32_t x[4];
-                q8w_widen4(d[2 * j], x[0], x[1]);
-                q8w_widen4(d[2 * j + 1], x[2], x[3]);
-                wq[t][j] = __builtin_bit_cast(bf16x8, (u32x4){x[0], x[1], x[2], x[3]});
-            }
-        }
-        if (kc + 1 < nk) {
-            load_a(kc + 1);
-            load_w(kc + 1);
-        }
-        const char *st = lds + (kc & 1) * STAGE;
+            for (int t = 0; t < TN; ++t) {
+                const uint32_t d[4] = {wr[b][t].x, wr[b][t].y, wr[b][t].z, wr[b][t].w};
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const char *fb = st + (TM * wm + i) * 6144 + j * 1024 + lane * 16;
-                const bf16x8 p1 = *reinterpret_cast<const bf16x8 *>(fb);
-                const bf16x8 p2 = *reinterpret_cast<const bf16x8 *>(fb + 2048);
-                const bf16x8 p3 = *reinterpret_cast<const bf16x8 *>(fb + 4096);
-#pragma unroll
-                for (int t = 0; t < TN; ++t) {
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p3, wq[t][j], acc[i][t], 0, 0, 0);
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p2, wq[t][j], acc[i][t], 0, 0, 0);
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p1, wq[t][j], acc[i][t], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) {
+                    uint32_t x[4];
+                    q8w_widen4(d[2 * j], x[0], x[1]);
+                    q8w_widen4(d[2 * j + 1], x[2], x[3]);
+                    wq[t][j] = __builtin_bit_cast(bf16x8, (u32x4){x[0], x[1], x[2], x[3]});
                 }
             }
-        if (kc + 1 < nk) store_a((kc + 1) & 1);  // that stage was last read before the previous barrier
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                bf16x8 p[TM][3];
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        p[i][q] = *reinterpret_cast<const bf16x8 *>(cur + q * PL + (32 * (TM * wm + i) + r) * P + 64 * b +
+                                                                    32 * hf + 16 * j);
+#pragma unroll
+                for (int q = 2; q >= 0; --q)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int t = 0; t < TN; ++t)
+                            acc[(2 * b + j) % NACC][i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                p[i][q], wq[t][j], acc[(2 * b + j) % NACC][i][t], 0, 0, 0);
+            }
+        }
+        load_w(min(c + 1, last));
+        store_a(c + 1, nxt);
+        load_a(min(c + 2, last));
         lds_barrier();
     }
-
-    // ---- C = acc * wscale[n]: lane holds channel n0 + 32 (TN wn + t) + lane % 32, rows acc_row
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
-        const int n = n0 + 32 * (TN * wn + t) + (lane & 31);
+        const int n = n0 + 32 * (TN * wn + t) + r;
         const float s = ws[min(n, N - 1)];
         if (n >= N) continue;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             const int mb = m0 + 32 * (TM * wm + i);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = mb + acc_row(r, lane);
-                if (m < M) C[(int64_t)m * ldc + n] = acc[i][t][r] * s;
+            for (int e = 0; e < 16; ++e) {
+                const int m = mb + acc_row(e, lane);
+                float v = acc[0][i][t][e];
+#pragma unroll
+                for (int a = 1; a < NACC; ++a) v += acc[a][i][t][e];
+                if (m < M) C[(int64_t)m * ldc + n] = v * s;
             }
         }
     }
 }
 
-// Small-M form: one workgroup per 32-row x (32 TN)-channel tile, its 4 wavefronts
+// Small form: one workgroup per 32-row x 32-channel tile, its 4 wavefronts
 // splitting K (wavefront w takes the 32-deep chunks w, w + 4, w + 8, ...). Each lane loads
 // its own MFMA operand values straight from HBM -- lane (row m, half h) the 16 activations
 // a[m, 32 kc + 16 h ..], split in registers, and its 16 weight bytes -- so there is no LDS
@@ -234,23 +228,21 @@ __global__ __launch_bounds__(256, 2) void gemm_q8w(const float *__restrict__ A, 
 // edges and preconditions as gemm_q8w.
 constexpr int Q8W_RING = 4;
 
-template <int TN, bool VEC>
+template <bool VEC>
 __global__ __launch_bounds__(256) void gemm_q8w_small(const float *__restrict__ A, int64_t lda,
                                                       const int8_t *__restrict__ W, const float *__restrict__ ws,
                                                       float *__restrict__ C, int64_t ldc, int M, int N, int K, int Kp,
                                                       int tilesN) {
-    __shared__ float red[4][TN][16][64];
+    __shared__ float red[4][16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
     const int logical = xcd_logical_tile(blockIdx.x, gridDim.x);
-    const int m0 = (logical / tilesN) * 32, n0 = (logical % tilesN) * (32 * TN);
+    const int m0 = (logical / tilesN) * 32, n0 = (logical % tilesN) * 32;
     const int nk = Kp / 32;
     const float *arow = A + (int64_t)min(m0 + (lane & 31), M - 1) * lda + 16 * h;
-    const int8_t *wb[TN];
-#pragma unroll
-    for (int t = 0; t < TN; ++t) wb[t] = W + ((int64_t)((n0 >> 5) + t) * nk) * 1024 + lane * 16;
+    const int8_t *wb = W + ((int64_t)(n0 >> 5) * nk) * 1024 + lane * 16;
 
     float av[Q8W_RING][16];
-    u32x4 wr[Q8W_RING][TN];
+    u32x4 wr[Q8W_RING];
     // chunk kc into ring slot d (kc < nk, uniform per wavefront)
     auto load = [&](int d, int kc) {
         const int k0 = 32 * kc + 16 * h;
@@ -275,15 +267,12 @@ __global__ __launch_bounds__(256) void gemm_q8w_small(const float *__restrict__ 
                 av[d][i] = k0 + i < K ? x : 0.0f;
             }
         }
-#pragma unroll
-        for (int t = 0; t < TN; ++t) wr[d][t] = *reinterpret_cast<const u32x4 *>(wb[t] + (int64_t)kc * 1024);
+        wr[d] = *reinterpret_cast<const u32x4 *>(wb + (int64_t)kc * 1024);
     };
 
-    f32x16 acc[TN];
+    f32x16 acc;
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[t][e] = 0.0f;
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
 
 #pragma unroll
     for (int d = 0; d < Q8W_RING; ++d)
@@ -307,49 +296,37 @@ __global__ __launch_bounds__(256) void gemm_q8w_small(const float *__restrict__ 
                 ap[2][j] = __builtin_bit_cast(bf16x8, (u32x4){q8w_pack(t3[0], t3[1]), q8w_pack(t3[2], t3[3]),
                                                               q8w_pack(t3[4], t3[5]), q8w_pack(t3[6], t3[7])});
             }
-            bf16x8 wq[TN][2];
+            bf16x8 wq[2];
+            const uint32_t dw[4] = {wr[d].x, wr[d].y, wr[d].z, wr[d].w};
 #pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                const uint32_t dw[4] = {wr[d][t].x, wr[d][t].y, wr[d][t].z, wr[d][t].w};
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    uint32_t x[4];
-                    q8w_widen4(dw[2 * j], x[0], x[1]);
-                    q8w_widen4(dw[2 * j + 1], x[2], x[3]);
-                    wq[t][j] = __builtin_bit_cast(bf16x8, (u32x4){x[0], x[1], x[2], x[3]});
-                }
+            for (int j = 0; j < 2; ++j) {
+                uint32_t x[4];
+                q8w_widen4(dw[2 * j], x[0], x[1]);
+                q8w_widen4(dw[2 * j + 1], x[2], x[3]);
+                wq[j] = __builtin_bit_cast(bf16x8, (u32x4){x[0], x[1], x[2], x[3]});
             }
             if (kc + 4 * Q8W_RING < nk) load(d, kc + 4 * Q8W_RING);
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int t = 0; t < TN; ++t) {
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[2][j], wq[t][j], acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[1][j], wq[t][j], acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[0][j], wq[t][j], acc[t], 0, 0, 0);
-                }
+                for (int q = 2; q >= 0; --q) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[q][j], wq[j], acc, 0, 0, 0);
         }
     }
 
     // ---- the four partial sums, added in wavefront order; wavefront w finishes the
-    // accumulator registers 4w .. 4w + 3 (rows acc_row(r, lane)) of every channel block
+    // accumulator registers 4w .. 4w + 3 (rows acc_row(r, lane))
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) red[wave][t][r][lane] = acc[t][r];
+    for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[r];
     __syncthreads();
+    const int n = n0 + (lane & 31);
+    const float s = ws[min(n, N - 1)];
+    if (n >= N) return;
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        const int n = n0 + 32 * t + (lane & 31);
-        const float s = ws[min(n, N - 1)];
-        if (n >= N) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 4 * wave + i;
-            const float v = ((red[0][t][r][lane] + red[1][t][r][lane]) + red[2][t][r][lane]) + red[3][t][r][lane];
-            const int m = m0 + acc_row(r, lane);
-            if (m < M) C[(int64_t)m * ldc + n] = v * s;
-        }
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * wave + i;
+        const float v = ((red[0][r][lane] + red[1][r][lane]) + red[2][r][lane]) + red[3][r][lane];
+        const int m = m0 + acc_row(r, lane);
+        if (m < M) C[(int64_t)m * ldc + n] = v * s;
     }
 }
 

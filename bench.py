@@ -645,8 +645,8 @@ def other_configs(ctx, torch, stream, ceilings):
         q8[f"m{M}_frac_bf16_mfma_peak"] = 3 * tot_flop / (tot_us * 1e-6) / PEAK_BF16_FLOPS
         if tot_host_us:
             q8[f"m{M}_layer_host_us"] = tot_host_us
-    q8.update({"kernels": "enchip::gemm_q8w<TM, TN, VEC> (LDS-staged split, 64 x 64 to 128 x 256 tiles), "
-                          "enchip::gemm_q8w_small<TN, VEC> (K split over the workgroup's wavefronts)",
+    q8.update({"kernels": "enchip::gemm_q8w<TM, TN, WM, WN, KC, NACC, VEC> (split planes in LDS, 32 x 128 or 128 x 256 "
+                          "tiles), enchip::gemm_q8w_small<VEC> (K split over the workgroup's wavefronts)",
                "note": "TFLOP/s = 2MNK / time; each f32 activation is split exactly into three bf16 parts, so the "
                        "bf16 MFMA fraction counts 3 x 2MNK; host_us includes the upload of a and download of dst"})
     out["matmul_bt_q8_weight_only"] = q8
