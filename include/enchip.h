@@ -23,7 +23,7 @@
  *   - The context's device scratch (the quantized activations of the entry points
  *     that quantize themselves, the top-k candidates) is shared by all of them. Work
  *     that uses it on one stream waits, on the device, for its last use on another
- *     stream (an event the library records after each such use), so host calls and
+ *     stream (through an event of the library), so host calls and
  *     *_dev calls on different streams may be mixed. Under HIP graph capture the
  *     library records no such event and the caller orders the streams.
  *
