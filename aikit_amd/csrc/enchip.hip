@@ -545,35 +545,56 @@ int skinny_nk(const enchip_ctx *c, const Weight &w, int64_t M, const void *aq, i
     return M > c->small_m && M <= 256 ? skinny_shape_nk(w, aq, lda, af) : 0;
 }
 
-template <int MB, int EPI, bool AF>
-void launch_skinny_mb(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq, int64_t lda, const float *as,
-                      const float *bias, float *out, int64_t ldo, int64_t M, hipStream_t s,
-                      const enchip::TopkSink &sink) {
-    using namespace enchip;
+dim3 skinny_grid(const enchip_ctx *c, const Weight &w) {
     const int64_t groups = (w.N + 31) / 32;
-    const dim3 grid((unsigned)std::min<int64_t>(c->num_cus, (groups + SK_WAVES - 1) / SK_WAVES)), block(64 * SK_WAVES);
-#define SK_CASE(NK)                                                                                                    \
-    case NK:                                                                                                           \
-        hipLaunchKernelGGL((gemm_w8a8_skinny<MB, NK, EPI, AF>), grid, block, 0, s, aq, lda, w.d_w, as, w.d_s, bias, \
-                           out, ldo, (int)M, (int)w.N, sink);                                                          \
-        break;
-    switch (nk) {
-        SK_CASE(4)
-        SK_CASE(8)
-        SK_CASE(12)
-        SK_CASE(16)
-        default: break;
+    return dim3((unsigned)std::min<int64_t>(c->num_cus, (groups + enchip::SK_WAVES - 1) / enchip::SK_WAVES));
+}
+
+#define SK_SWITCH(nk)   \
+    switch (nk) {       \
+        SK_CASE(4)      \
+        SK_CASE(8)      \
+        SK_CASE(12)     \
+        SK_CASE(16)     \
+        default: break; \
     }
+
+template <int MB, bool AF>
+void launch_skinny_mb(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq, int64_t lda, const float *as,
+                      const float *bias, float *out, int64_t ldo, int64_t M, hipStream_t s) {
+    using namespace enchip;
+    const dim3 grid = skinny_grid(c, w), block(64 * SK_WAVES);
+#define SK_CASE(NK)                                                                                               \
+    case NK:                                                                                                      \
+        hipLaunchKernelGGL((gemm_w8a8_skinny<MB, NK, AF>), grid, block, 0, s, aq, lda, w.d_w, as, w.d_s, bias,    \
+                           out, ldo, (int)M, (int)w.N);                                                           \
+        break;
+    SK_SWITCH(nk)
 #undef SK_CASE
 }
 
+// The top-k candidates of M <= 32 MB rows.
+template <int MB, int HB, int TN, int AHEAD>
+void launch_skinny_topk(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq, const float *as, int64_t M,
+                        hipStream_t s, const enchip::TopkSink &sink) {
+    using namespace enchip;
+    const dim3 grid = skinny_grid(c, w), block(64 * SK_WAVES);
+#define SK_CASE(NK)                                                                                                \
+    case NK:                                                                                                       \
+        hipLaunchKernelGGL((gemm_w8a8_skinny_topk<MB, NK, HB, TN, AHEAD>), grid, block, 0, s, aq, w.d_w, as,       \
+                           w.d_s, (int)M, (int)w.N, sink);                                                         \
+        break;
+    SK_SWITCH(nk)
+#undef SK_CASE
+}
+#undef SK_SWITCH
+
 // nk from skinny_nk; 32 x 4 or 32 x 8 rows staged.
-template <int EPI, bool AF>
+template <bool AF>
 void launch_skinny(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq, int64_t lda, const float *as,
-                   const float *bias, float *out, int64_t ldo, int64_t M, hipStream_t s,
-                   const enchip::TopkSink &sink = {}) {
-    if (M <= 128) launch_skinny_mb<4, EPI, AF>(c, w, nk, aq, lda, as, bias, out, ldo, M, s, sink);
-    else launch_skinny_mb<8, EPI, AF>(c, w, nk, aq, lda, as, bias, out, ldo, M, s, sink);
+                   const float *bias, float *out, int64_t ldo, int64_t M, hipStream_t s) {
+    if (M <= 128) launch_skinny_mb<4, AF>(c, w, nk, aq, lda, as, bias, out, ldo, M, s);
+    else launch_skinny_mb<8, AF>(c, w, nk, aq, lda, as, bias, out, ldo, M, s);
 }
 
 // Piece sizes as kPieces. pt: gemm_w8a8_pt's outputs (16-byte stores), else any.
@@ -600,8 +621,8 @@ bool launch_gemm_epi(enchip_ctx *c, const Weight &w, const int8_t *aq, int64_t l
                      const float *bias, void *out, int64_t ldo, int64_t M, hipStream_t s, bool af) {
     if (EPI == enchip::EPI_F32) {
         if (const int nk = skinny_nk(c, w, M, aq, lda, af)) {
-            if (af) launch_skinny<enchip::EPI_F32, true>(c, w, nk, aq, lda, as, bias, (float *)out, ldo, M, s);
-            else launch_skinny<enchip::EPI_F32, false>(c, w, nk, aq, lda, as, bias, (float *)out, ldo, M, s);
+            if (af) launch_skinny<true>(c, w, nk, aq, lda, as, bias, (float *)out, ldo, M, s);
+            else launch_skinny<false>(c, w, nk, aq, lda, as, bias, (float *)out, ldo, M, s);
             return true;
         }
     }
@@ -855,7 +876,7 @@ int enchip_gemm_kernel_name(enchip_ctx *ctx, enchip_weight h, int64_t M, int act
     char name[96];
     const int sk = epi == enchip::EPI_F32 ? skinny_nk(ctx, *w, M, nullptr, w->Kp, true) : 0;
     if (sk)  // the library's own quantization is fragment-major (pre_dev's row-major codes: false)
-        snprintf(name, sizeof name, "enchip::gemm_w8a8_skinny<%d, %d, %d, true>", M <= 128 ? 4 : 8, sk, epi);
+        snprintf(name, sizeof name, "enchip::gemm_w8a8_skinny<%d, %d, true>", M <= 128 ? 4 : 8, sk);
     else if (const bool pt = route_af(ctx, *w, M, nullptr, w->N); pt || route_frag(ctx, *w, M, epi, nullptr, w->N)) {
         const int f = piece_form(ctx, *w, M, epi, !pt);
         if (f >= 0 && pt)
@@ -2114,22 +2135,25 @@ int launch_ann_fused(enchip_ctx *c, const Weight &w, int64_t M, int64_t k, hipSt
     sink.score = raw;
     sink.cap = (int)cap;
     if (const int nk = skinny_shape_nk(w, c->d_aq, w.Kp, true)) {
-        // 128 rows a launch, whatever M (each launch reads the index once): with 256 rows'
-        // accumulators the candidate epilogue spills, and at M = 1024 eight launches took
-        // well under the persistent kernel's candidate pass
-        for (int64_t r0 = 0; r0 < M; r0 += 128) {
+        // 256 rows a launch (each reads the index once) while a row lists in one workgroup, as
+        // expected, half of its LDS slots there or less (k N / kSinkSample / workgroups); past
+        // that every other candidate would go to the global lists one by one. Measured on MI355X
+        // (256 queries, 2^20 x 384, per host call): k = 32 (4 of 8 slots) 346 -> 298 us against two
+        // launches of 128 rows, k = 64 (8 of 8) 416 -> 431.
+        const int64_t slots = kSinkSample * (int64_t)skinny_grid(c, w).x;
+        const int64_t most = 2 * k * w.N <= sk_lcap(8) * slots ? 256 : 128;
+        for (int64_t r0 = 0; r0 < M; r0 += most) {
             TopkSink part = sink;
             part.thr += r0;
             part.count += r0;
             part.key += r0 * cap;
             part.score += r0 * cap;
-            const int64_t mr = std::min<int64_t>(128, M - r0);
-            if (mr <= 32)  // one row block: the epilogue's work per score covers 32 rows, not 128
-                launch_skinny_mb<1, EPI_TOPK, true>(c, w, nk, c->d_aq + r0 * w.Kp, w.Kp, c->d_as + r0, nullptr,
-                                                    nullptr, 0, mr, s, part);
-            else
-                launch_skinny_mb<4, EPI_TOPK, true>(c, w, nk, c->d_aq + r0 * w.Kp, w.Kp, c->d_as + r0, nullptr,
-                                                    nullptr, 0, mr, s, part);
+            const int64_t mr = std::min<int64_t>(most, M - r0);
+            const int8_t *aq = c->d_aq + r0 * w.Kp;
+            const float *as = c->d_as + r0;
+            if (mr <= 32) launch_skinny_topk<1, 1, 1, 2>(c, w, nk, aq, as, mr, s, part);
+            else if (mr <= 128) launch_skinny_topk<4, 2, 1, 2>(c, w, nk, aq, as, mr, s, part);
+            else launch_skinny_topk<8, 1, 2, 3>(c, w, nk, aq, as, mr, s, part);
         }
     } else
         launch_pt<PT_PW, EPI_TOPK, true>(c, w, c->d_aq, w.Kp, c->d_as, nullptr, nullptr, 0, M, s, sink);

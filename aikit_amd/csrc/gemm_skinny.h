@@ -1,6 +1,6 @@
 // gemm_skinny.h -- W8A8 for a few rows against very many output channels with a short K:
 // ann.FlatI8 scoring (M queries x an index of n rows, ann/backend.go:16-60) and its
-// fused top-k. gemm_w8a8_skinny.
+// fused top-k: gemm_w8a8_skinny (the scores) and gemm_w8a8_skinny_topk (their candidates).
 //
 // The persistent tiled kernel (gemm_persistent.h) streams the weights once per 128-row
 // block, and at a short K each tile brings only its ring's stages of weights in flight: at
@@ -15,9 +15,9 @@
 //   * per group, MB x NK v_mfma_i32_32x32x32_i8 (one per row block and K step) read
 //     their A fragments from LDS;
 //   * the epilogue works on the accumulators in place (a lane holds one channel of 16
-//     rows per row block): EPI_F32 stores the dequantized values (32 lanes write 128
-//     contiguous bytes of a row); EPI_TOPK compares them with the rows' bounds and lists
-//     the few at or above them (TopkSink), storing nothing else.
+//     rows per row block): the dequantized values are stored (32 lanes write 128
+//     contiguous bytes of a row), or compared with the rows' bounds, the few at or above
+//     them listed (TopkSink) and nothing else stored.
 // Numerics: the exact int32 dot and the dequantization of the other kernels, so the
 // outputs are bit-identical to theirs.
 #pragma once
@@ -36,30 +36,18 @@
 namespace enchip {
 
 constexpr int SK_WAVES = 8;  // waves per workgroup, one workgroup per CU
-constexpr int SK_LCAP = 16;  // EPI_TOPK: candidates per row a workgroup holds in LDS
 
 // MB: row blocks staged (32 * MB >= M; fragment-major A is read up to 32 * MB rows, which
 // its buffer holds: it is padded to a multiple of 128 rows and MB is 4 or 8). NK = Kp / 32.
 // AF: A is fragment-major ([M/32][NK][1024]); otherwise row-major int8 at pitch lda (a
 // multiple of 16, at least Kp, zero past K).
-template <int MB, int NK, int EPI, bool AF>
+template <int MB, int NK, bool AF>
 __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
     const int8_t *__restrict__ A, int64_t lda, const int8_t *__restrict__ Wf, const float *__restrict__ aS,
     const float *__restrict__ wS, const float *__restrict__ bias, float *__restrict__ out, int64_t ldo, int M,
-    int N, TopkSink sink) {
-    static_assert(EPI == EPI_F32 || EPI == EPI_TOPK, "f32 scores or their top-k candidates");
+    int N) {
     __shared__ i32x4 s_a[MB * NK * 64];
     __shared__ __attribute__((aligned(16))) float s_as[MB * 32];
-    __shared__ uint64_t s_thr[EPI == EPI_TOPK ? MB * 32 : 1];
-    __shared__ __attribute__((aligned(16))) float s_tf[EPI == EPI_TOPK ? MB * 32 : 1];  // bound scores
-    // EPI_TOPK: the workgroup's candidates, per row, until its flush at the end. A global
-    // atomic that returns its value would wait (in-order vmcnt) for every weight load in
-    // flight behind it, a full memory latency per group with a candidate; LDS atomics
-    // count on lgkmcnt.
-    constexpr int LC = EPI == EPI_TOPK ? MB * 32 : 1;
-    __shared__ unsigned s_cnt[LC];
-    __shared__ uint64_t s_ckey[LC * SK_LCAP];
-    __shared__ float s_cscore[LC * SK_LCAP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
     // A fragment f = rb * NK + kk holds, in lane l, row 32 rb + (l & 31), bytes
@@ -73,55 +61,34 @@ __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
             s_a[i] = *reinterpret_cast<const i32x4 *>(A + (int64_t)row * lda + kk * 32 + (l >> 5) * 16);
         }
     }
-    for (int r = tid; r < MB * 32; r += 64 * SK_WAVES) {
-        s_as[r] = aS[min(r, M - 1)];
-        if (EPI == EPI_TOPK) {
-            const uint64_t t = sink.thr[min(r, M - 1)];
-            s_thr[r] = t;
-            s_tf[r] = t == 0 ? -INFINITY : topk_key_score(t);  // -inf: no bound, every non-NaN score
-            s_cnt[r] = 0;
-        }
-    }
+    for (int r = tid; r < MB * 32; r += 64 * SK_WAVES) s_as[r] = aS[min(r, M - 1)];
     __syncthreads();
 
     const int groups = (N + 31) >> 5, stride = gridDim.x * SK_WAVES;
     int g = blockIdx.x * SK_WAVES + wave;
-    if (EPI != EPI_TOPK && g >= groups) return;  // no barrier follows
+    if (g >= groups) return;  // no barrier follows
     const int8_t *wl = Wf + lane * 16;
     auto wfrag = [&](int grp, int kk) {
         return __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(wl + ((int64_t)grp * NK + kk) * 1024));
     };
     auto chan = [&](int grp) { return min(grp * 32 + (lane & 31), N - 1); };
     const bool has_bias = bias != nullptr;
-    // The weight ring: D groups of NK fragments, each slot refilled with the group D ahead
-    // while its current group's MFMAs issue. Two slots where the registers allow (the
-    // candidate epilogue, up to 4 row blocks and 12 K steps): with one, 2 waves per SIMD x
-    // 12 KiB in flight left the index streaming at ~3 TB/s (latency-bound). The f32
-    // epilogue keeps one: its stores, not the index, bound it.
-    constexpr int D = EPI == EPI_TOPK && MB <= 4 && NK <= 12 ? 2 : 1;
-    i32x4 b[D][NK];
-    float wsr[D], bbr[D];
-    const int n = g < groups ? (groups - 1 - g) / stride + 1 : 0;  // this wave's groups
+    i32x4 b[NK];  // each refilled with the next group's fragment while this one's MFMAs issue
+    const int n = (groups - 1 - g) / stride + 1;  // this wave's groups
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        const int gd = min(g + d * stride, groups - 1);  // in bounds also past the wave's groups
-#pragma unroll
-        for (int kk = 0; kk < NK; ++kk) b[d][kk] = wfrag(gd, kk);
-        wsr[d] = wS[chan(gd)];
-        bbr[d] = has_bias ? bias[chan(gd)] : kNoBias;
-    }
+    for (int kk = 0; kk < NK; ++kk) b[kk] = wfrag(g, kk);
+    float ws_n = wS[chan(g)], bb_n = has_bias ? bias[chan(g)] : kNoBias;
 
-    // Group i of this wave from ring slot SLOT: its MFMAs (each K step's MB A fragments read
-    // from LDS first, then its MB MFMAs, then, with NEXT, the fragment of that step of group
-    // i + D: a fixed order, so only one step's A fragments are live), then its epilogue.
-    auto group = [&](auto slot_c, auto next_c, int i) {
-        constexpr int SLOT = decltype(slot_c)::value;
+    // Group i of this wave: its MFMAs (each K step's MB A fragments read from LDS first, then
+    // its MB MFMAs, then, with NEXT, the fragment of that step of group i + 1: a fixed order,
+    // so only one step's A fragments are live), then its epilogue.
+    auto group = [&](auto next_c, int i) {
         constexpr bool NEXT = decltype(next_c)::value;
-        const int g = blockIdx.x * SK_WAVES + wave + i * stride, gn = g + D * stride;
-        const float ws_c = wsr[SLOT], bb_c = bbr[SLOT];
+        const int g = blockIdx.x * SK_WAVES + wave + i * stride, gn = g + stride;
+        const float ws_c = ws_n, bb_c = bb_n;
         if (NEXT) {
-            wsr[SLOT] = wS[chan(gn)];
-            bbr[SLOT] = has_bias ? bias[chan(gn)] : kNoBias;
+            ws_n = wS[chan(gn)];
+            bb_n = has_bias ? bias[chan(gn)] : kNoBias;
         }
         i32x16 acc[MB];
 #pragma unroll
@@ -135,8 +102,8 @@ __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
             for (int rb = 0; rb < MB; ++rb) af[rb] = s_a[(rb * NK + kk) * 64 + lane];
 #pragma unroll
             for (int rb = 0; rb < MB; ++rb)
-                acc[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[rb], b[SLOT][kk], acc[rb], 0, 0, 0);
-            if (NEXT) b[SLOT][kk] = wfrag(gn, kk);
+                acc[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[rb], b[kk], acc[rb], 0, 0, 0);
+            if (NEXT) b[kk] = wfrag(gn, kk);
             __builtin_amdgcn_sched_group_barrier(0x100, MB, 0);  // LDS reads
             __builtin_amdgcn_sched_group_barrier(0x008, MB, 0);  // MFMAs
             if (NEXT) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // the VMEM load
@@ -144,68 +111,182 @@ __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
 
         const int col = g * 32 + (lane & 31);
         if (col >= N) return;  // the ragged last group
-        // The output rows' offsets and the candidate lists' addresses depend only on the
-        // lane: left to itself the compiler computes all MB x 16 of them once, before the
-        // group loop, and spills. An opaque copy of the pitch (and of the row in the rare
-        // path) keeps each one next to its use.
+        // The output rows' offsets depend only on the lane: left to itself the compiler
+        // computes all MB x 16 of them once, before the group loop, and spills. An opaque copy
+        // of the pitch keeps each one next to its use.
         int64_t ld = ldo;
         asm volatile("" : "+s"(ld));
-        if constexpr (EPI == EPI_F32) {
 #pragma unroll
-            for (int rb = 0; rb < MB; ++rb)
+        for (int rb = 0; rb < MB; ++rb)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int row0 = rb * 32 + 8 * q + 4 * (lane >> 5);  // rows row0 .. row0 + 3
+                const float4 as4 = *reinterpret_cast<const float4 *>(&s_as[row0]);
+                const float asv[4] = {as4.x, as4.y, as4.z, as4.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (row0 + u < M)
+                        __builtin_nontemporal_store(dequant(acc[rb][4 * q + u], asv[u], ws_c, bb_c),
+                                                    out + (int64_t)(row0 + u) * ld + col);
+            }
+    };
+    for (int i = 0; i + 1 < n; ++i) group(std::true_type{}, i);
+    group(std::false_type{}, n - 1);
+}
+
+// The scores' top-k candidates (TopkSink) instead of the scores, on fragment-major A. A wave
+// takes TN 32-channel groups at a time and their row blocks HB by HB, the A fragments of K step
+// kk + AHEAD in flight from LDS while step kk's MFMAs issue; the last row blocks' MFMAs refill
+// the weight fragments, which then have those blocks' epilogue and the next group's start to
+// arrive in.
+//
+// A score is compared by one multiply: (float)acc * ws against s_low, a lower bound of the
+// row's bound score divided by the row's scale. With y = acc * ws in f32, x the score
+// ((float)acc * as) * ws and tf the bound, x >= tf implies y >= (tf - 2^-20 |tf| - 2^-100) / as
+// for 2^-100 <= as <= 2^40: rounding moves x from the product of the three by under 2^-22 of it
+// plus 2^-149 (subnormal products), y by 2^-24 of it plus 2^-150, and the bound leaves 2^-20 |tf|
+// and 2^-100 for both. Rows of another scale (0 and NaN included) or of no bound, and scores
+// whose y is NaN, take the exact test, as every score past the bound does: the dequantized score
+// and its key. Those are few, so the common path is a conversion, a multiply and a comparison
+// per score, where dequantizing and comparing each took six operations.
+//
+// The candidates of a workgroup wait in LDS until its end: a global atomic that returns its
+// value would wait (in-order vmcnt) for every weight load in flight behind it, LDS atomics
+// count on lgkmcnt.
+//
+// Up to 256 rows read the index once. Bound by the MFMA pipes and the LDS reads that feed them
+// (each A fragment read feeds TN MFMAs). Measured on MI355X over a 2^20 x 384 index, k = 10, per
+// pass: 256 rows 192 us (two passes of 128) -> 120, 129 rows 165 -> 104, 100 rows 89 -> 70, 16
+// rows 63 -> 61.
+constexpr int sk_lcap(int mb) { return mb > 4 ? 8 : 16; }  // candidates per row held in LDS
+
+template <int MB, int NK, int HB, int TN, int AHEAD>
+__global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny_topk(
+    const int8_t *__restrict__ A, const int8_t *__restrict__ Wf, const float *__restrict__ aS,
+    const float *__restrict__ wS, int M, int N, TopkSink sink) {
+    static_assert(MB % HB == 0 && AHEAD < NK, "whole parts");
+    constexpr int LCAP = sk_lcap(MB);
+    __shared__ i32x4 s_a[MB * NK * 64];
+    __shared__ __attribute__((aligned(16))) float s_as[MB * 32];
+    __shared__ uint64_t s_thr[MB * 32];
+    __shared__ __attribute__((aligned(16))) float s_low[MB * 32];
+    __shared__ unsigned s_cnt[MB * 32];
+    __shared__ uint64_t s_ckey[MB * 32 * LCAP];
+    __shared__ float s_cscore[MB * 32 * LCAP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < MB * NK * 64; i += 64 * SK_WAVES) s_a[i] = reinterpret_cast<const i32x4 *>(A)[i];
+    for (int r = tid; r < MB * 32; r += 64 * SK_WAVES) {
+        const float as = aS[min(r, M - 1)];
+        const uint64_t t = sink.thr[min(r, M - 1)];
+        s_as[r] = as;
+        s_thr[r] = t;
+        s_cnt[r] = 0;
+        const float tf = topk_key_score(t);
+        const bool exact = t == 0 || !(as >= 0x1p-100f && as <= 0x1p40f);
+        s_low[r] = r >= M ? INFINITY : exact ? -INFINITY : (tf - fabsf(tf) * 0x1p-20f - 0x1p-100f) / as;
+    }
+    __syncthreads();
+    const int groups = (N + 32 * TN - 1) / (32 * TN), stride = gridDim.x * SK_WAVES;
+    const int g0 = blockIdx.x * SK_WAVES + wave;
+    const int8_t *wl = Wf + lane * 16;
+    auto wfrag = [&](int cg, int kk) {
+        return __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(wl + ((int64_t)cg * NK + kk) * 1024));
+    };
+    auto wscale = [&](int cg) { return wS[min(cg * 32 + (lane & 31), N - 1)]; };
+    i32x4 b[TN][NK];
+    float wsr[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        const int cg = min(g0, groups - 1) * TN + t;
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) b[t][kk] = wfrag(cg, kk);
+        wsr[t] = wscale(cg);
+    }
+    for (int g = g0; g < groups; g += stride) {
+        const int gn = min(g + stride, groups - 1);
+        float ws[TN];
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            ws[t] = wsr[t];
+            wsr[t] = wscale(gn * TN + t);
+        }
+#pragma unroll
+        for (int h = 0; h < MB; h += HB) {
+            i32x16 acc[HB][TN];
+#pragma unroll
+            for (int rb = 0; rb < HB; ++rb)
+#pragma unroll
+                for (int t = 0; t < TN; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[rb][t][r] = 0;
+            i32x4 af[AHEAD + 1][HB];
+#pragma unroll
+            for (int p = 0; p < AHEAD; ++p)
+#pragma unroll
+                for (int rb = 0; rb < HB; ++rb) af[p][rb] = s_a[((h + rb) * NK + p) * 64 + lane];
+#pragma unroll
+            for (int kk = 0; kk < NK; ++kk) {
+                if (kk + AHEAD < NK)
+#pragma unroll
+                    for (int rb = 0; rb < HB; ++rb)
+                        af[(kk + AHEAD) % (AHEAD + 1)][rb] = s_a[((h + rb) * NK + kk + AHEAD) * 64 + lane];
+#pragma unroll
+                for (int rb = 0; rb < HB; ++rb)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t)
+                        acc[rb][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[kk % (AHEAD + 1)][rb], b[t][kk], acc[rb][t], 0, 0, 0);
+                if (h + HB >= MB)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) b[t][kk] = wfrag(gn * TN + t, kk);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int rb = 0; rb < HB; ++rb) {
+                bool pass[TN];
+#pragma unroll
+                for (int t = 0; t < TN; ++t) pass[t] = false;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int row0 = rb * 32 + 8 * q + 4 * (lane >> 5);  // rows row0 .. row0 + 3
-                    const float4 as4 = *reinterpret_cast<const float4 *>(&s_as[row0]);
-                    const float asv[4] = {as4.x, as4.y, as4.z, as4.w};
+                    const float4 lo4 = *reinterpret_cast<const float4 *>(&s_low[(h + rb) * 32 + 8 * q + 4 * (lane >> 5)]);
+                    const float lo[4] = {lo4.x, lo4.y, lo4.z, lo4.w};
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
-                        if (row0 + u < M)
-                            __builtin_nontemporal_store(dequant(acc[rb][4 * q + u], asv[u], ws_c, bb_c),
-                                                        out + (int64_t)(row0 + u) * ld + col);
+#pragma unroll
+                        for (int t = 0; t < TN; ++t) pass[t] |= !((float)acc[rb][t][4 * q + u] * ws[t] < lo[u]);
                 }
-        } else {
-            const uint32_t lo = 0xffffffffu - (uint32_t)col;
 #pragma unroll
-            for (int rb = 0; rb < MB; ++rb) {
-                // bit 4q + u: value acc[rb][4q + u] is at or above its row's bound score (a
-                // NaN is not), which a kept key needs; only ties at that score need the
-                // index test below
-                uint32_t pass = 0;
+                for (int t = 0; t < TN; ++t) {
+                    const int col = (g * TN + t) * 32 + (lane & 31);
+                    if (pass[t] && col < N) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int row0 = rb * 32 + 8 * q + 4 * (lane >> 5);
-                    const float4 as4 = *reinterpret_cast<const float4 *>(&s_as[row0]);
-                    const float4 tf4 = *reinterpret_cast<const float4 *>(&s_tf[row0]);
-                    const float asv[4] = {as4.x, as4.y, as4.z, as4.w}, tfv[4] = {tf4.x, tf4.y, tf4.z, tf4.w};
+                        for (int q = 0; q < 4; ++q) {
+                            int row0 = (h + rb) * 32 + 8 * q + 4 * (lane >> 5);
+                            asm volatile("" : "+v"(row0));  // else every row's addresses live across the loop
+                            const float4 lo4 = *reinterpret_cast<const float4 *>(&s_low[row0]);
+                            const float lo[4] = {lo4.x, lo4.y, lo4.z, lo4.w};
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        pass |= dequant(acc[rb][4 * q + u], asv[u], ws_c, bb_c) >= tfv[u] ? 1u << (4 * q + u) : 0u;
-                }
-                if (pass != 0u) {  // rare: the exact key test
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        if (!((pass >> r) & 1u)) continue;
-                        int row = rb * 32 + acc_row(r, lane);
-                        asm volatile("" : "+v"(row));
-                        const float x = dequant(acc[rb][r], s_as[row], ws_c, bb_c);
-                        const uint64_t t = s_thr[row];
-                        const float tf = topk_key_score(t);
-                        // key >= t: the score above t's, or equal and the index no larger;
-                        // t == 0 keeps every non-NaN score
-                        const bool in = row < M && (t == 0 || x > tf || (x == tf && lo >= (uint32_t)t)) && x == x;
-                        if (in) {
-                            const uint64_t key = ((uint64_t)topk_order(x) << 32) | lo;
-                            const unsigned p = atomicAdd(&s_cnt[row], 1u);
-                            if (p < (unsigned)SK_LCAP) {
-                                s_ckey[row * SK_LCAP + p] = key;
-                                s_cscore[row * SK_LCAP + p] = x;
-                            } else {  // the row's LDS slots are full: straight to its list
-                                const unsigned pos = atomicAdd(&sink.count[row], 1u);
-                                if (pos < (unsigned)sink.cap) {
-                                    const int64_t at = (int64_t)row * sink.cap + pos;
-                                    sink.key[at] = key;
-                                    sink.score[at] = x;
+                            for (int u = 0; u < 4; ++u) {
+                                if ((float)acc[rb][t][4 * q + u] * ws[t] < lo[u]) continue;
+                                const int row = row0 + u;
+                                const float x = dequant(acc[rb][t][4 * q + u], s_as[row], ws[t], kNoBias);
+                                // key >= tk: the score above tk's, or equal and the index no
+                                // larger; tk == 0 keeps every non-NaN score
+                                const uint64_t key = ((uint64_t)topk_order(x) << 32) | (0xffffffffu - (uint32_t)col);
+                                const uint64_t tk = s_thr[row];
+                                const float tf = topk_key_score(tk);
+                                if (row < M && x == x && (tk == 0 || x > tf || (x == tf && (uint32_t)key >= (uint32_t)tk))) {
+                                    const unsigned at_l = atomicAdd(&s_cnt[row], 1u);
+                                    if (at_l < (unsigned)LCAP) {
+                                        s_ckey[row * LCAP + at_l] = key;
+                                        s_cscore[row * LCAP + at_l] = x;
+                                    } else {  // the row's LDS slots are full: straight to its list
+                                        const unsigned pos = atomicAdd(&sink.count[row], 1u);
+                                        if (pos < (unsigned)sink.cap) {
+                                            const int64_t at = (int64_t)row * sink.cap + pos;
+                                            sink.key[at] = key;
+                                            sink.score[at] = x;
+                                        }
+                                    }
                                 }
                             }
                         }
@@ -214,45 +295,19 @@ __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
                 __builtin_amdgcn_sched_barrier(0);  // one row block at a time
             }
         }
-    };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, D - 1>;
-    using T = std::true_type;
-    using F = std::false_type;
-    int i = 0;
-    if constexpr (D == 2) {
-        for (; i + 3 < n; i += 2) {
-            group(S0{}, T{}, i);
-            group(S1{}, T{}, i + 1);
-        }
-        if (n - i == 3) {
-            group(S0{}, T{}, i);
-            group(S1{}, F{}, i + 1);
-            group(S0{}, F{}, i + 2);
-        } else if (n - i == 2) {
-            group(S0{}, F{}, i);
-            group(S1{}, F{}, i + 1);
-        } else if (n - i == 1) {
-            group(S0{}, F{}, i);
-        }
-    } else {
-        for (; i + 1 < n; ++i) group(S0{}, T{}, i);
-        if (n - i == 1) group(S0{}, F{}, i);
     }
-    if constexpr (EPI == EPI_TOPK) {
-        // flush: one global atomic per row that holds candidates reserves their places
-        __syncthreads();
-        for (int r = tid; r < M && r < MB * 32; r += 64 * SK_WAVES) {
-            const unsigned n = min(s_cnt[r], (unsigned)SK_LCAP);
-            if (n == 0) continue;
-            const unsigned base = atomicAdd(&sink.count[r], n);
-            for (unsigned i = 0; i < n; ++i)
-                if (base + i < (unsigned)sink.cap) {
-                    const int64_t at = (int64_t)r * sink.cap + base + i;
-                    sink.key[at] = s_ckey[r * SK_LCAP + i];
-                    sink.score[at] = s_cscore[r * SK_LCAP + i];
-                }
-        }
+    // flush: one global atomic per row that holds candidates reserves their places
+    __syncthreads();
+    for (int r = tid; r < M && r < MB * 32; r += 64 * SK_WAVES) {
+        const unsigned n = min(s_cnt[r], (unsigned)LCAP);
+        if (n == 0) continue;
+        const unsigned base = atomicAdd(&sink.count[r], n);
+        for (unsigned i = 0; i < n; ++i)
+            if (base + i < (unsigned)sink.cap) {
+                const int64_t at = (int64_t)r * sink.cap + base + i;
+                sink.key[at] = s_ckey[r * LCAP + i];
+                sink.score[at] = s_cscore[r * LCAP + i];
+            }
     }
 }
 

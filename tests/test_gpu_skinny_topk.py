@@ -1,0 +1,51 @@
+"""GPU tests of the candidate kernel behind the fused top-k at its edges: against the oracle's
+scores and the reference's selection, exactly (ids, order and score bits)."""
+import numpy as np
+import oracle
+import pytest
+
+from aikit_amd import workloads
+
+pytestmark = pytest.mark.gpu
+
+
+# rows: one, two, four and eight row blocks a launch, ragged; a launch of one row after 256.
+# K: 4, 8, 12 and 16 K steps. N % 64 in {0, 4, 36}: the last pair of channel groups ragged.
+# k = 1, and 64 (a workgroup's slots for a row overflow into the global lists).
+@pytest.mark.parametrize("M,N,K,k", [(33, 131072, 128, 10), (128, 131076, 256, 1), (129, 131108, 384, 10),
+                                     (256, 131076, 512, 10), (257, 150004, 100, 10), (200, 262144, 384, 64),
+                                     (8, 131108, 512, 64)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_candidates_match_oracle(ctx, M, N, K, k, odd):
+    # odd: query rows of zeros and of scales outside the fast comparison's range (codes of
+    # subnormal and of very large values), index scales that are negative, zero, infinite, NaN,
+    # subnormal, and sign-flipped copies of index rows (ties of both signs).
+    g = workloads.rng(7100 + M + N + K + k)
+    q = workloads.activations(g, M, K)
+    codes = g.integers(-127, 128, size=(N, K), dtype=np.int8)
+    scales = g.uniform(1e-3, 1e-2, size=N).astype(np.float32)
+    if odd:
+        q[0] = 0
+        q[M // 2] *= np.float32(2.0 ** -110)
+        q[M - 1] *= np.float32(2.0 ** 60)
+        scales[g.random(N) < 0.2] *= -1
+        for v in (0.0, np.inf, -np.inf, np.nan, 1e-42):
+            scales[g.random(N) < 2e-5] = v
+        codes[N // 2:N // 2 + 4096] = -codes[:4096]
+        scales[N // 2:N // 2 + 4096] = -scales[:4096]
+    print(f"[case] skinny candidates M={M} N={N} K={K} k={k} odd={odd}", flush=True)
+    w = ctx.register_weight(codes, scales)
+    try:
+        f0, _ = ctx.ann_topk_stats()
+        hi, hs = ctx.ann_topk(w, q, k)
+        f1, _ = ctx.ann_topk_stats()
+    finally:
+        ctx.release_weight(w)
+    assert f1 == f0 + 1, "route"
+    with np.errstate(all="ignore"):
+        scores = oracle.w8a8_linear(q, codes, scales, None, 0, M, K, N)
+    for r in range(M):
+        idx, sc = oracle.top_hits(scores[r], k)
+        assert hi[r, :idx.size].tolist() == idx.tolist(), f"row {r}: indices differ"
+        assert np.array_equal(hs[r, :idx.size].view(np.uint32), sc.view(np.uint32)), f"row {r}: scores differ"
+        assert (hi[r, idx.size:] == -1).all() and np.isnan(hs[r, idx.size:]).all(), f"row {r}: padding"
