@@ -1879,7 +1879,8 @@ int enchip_pool_mean_l2_dev(enchip_ctx *ctx, const float *d_h, int64_t ldh, int6
     if (!d_out || (L > 0 && !d_h)) return fail(ctx, ENCHIP_ERR_ARG, "pool: null pointer");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    hipLaunchKernelGGL(enchip::pool_mean_cols, dim3((unsigned)((D + 255) / 256), (unsigned)nseq), dim3(256), 0, s, d_h,
+    hipLaunchKernelGGL(enchip::pool_mean_cols, dim3((unsigned)((D + enchip::POOL_COLS - 1) / enchip::POOL_COLS), (unsigned)nseq),
+                       dim3(enchip::POOL_COLS), 0, s, d_h,
                        ldh, (int)L, (int)D, d_out, ldo);
     hipLaunchKernelGGL(enchip::l2_normalize_rows, dim3((unsigned)nseq), dim3(256), 0, s, d_out, ldo, (int)D);
     return check_launch(ctx, "pool_mean_l2");

@@ -407,37 +407,69 @@ __global__ __launch_bounds__(256) void embed_rows(const int32_t *__restrict__ id
 // (encoder/pooling.go:84-105 poolOne(mean), embed/pool.go:22-38 L2Normalize) in the
 // reference's summation order, so the result is exact:
 //   pool_mean_cols: one thread per (sequence, column); the column's float64 sum runs over
-//     the rows in order; out = float32(sum * (1/L)). Grid (ceil(D/256), nseq).
-//   l2_normalize_rows: one block per sequence (D <= 4096); the row is staged in LDS, one
-//     thread adds the squares over the columns in order, then out = float32(out / norm),
-//     or 0 when norm < 1e-12.
-__global__ __launch_bounds__(256) void pool_mean_cols(const float *__restrict__ h, int64_t ldh, int L, int D,
-                                                      float *__restrict__ out, int64_t ldo) {
-    const int j = blockIdx.x * 256 + threadIdx.x;
+//     the rows in order; out = float32(sum * (1/L)). Grid (ceil(D/64), nseq).
+//   l2_normalize_rows: one block per sequence (D <= 4096); the squares in LDS, one thread
+//     adds them over the columns in order, then out = float32(out / norm), or 0 when
+//     norm < 1e-12.
+// Both are latency chains. The pooling's is one memory round trip per batch of loads: one
+// wavefront per block spreads the columns over the CUs and 32 rows' loads go out at once.
+// The norm's is one float64 add per column; the other threads prepare the squares, padded
+// with zeros (adding +0 to a sum of squares changes nothing, NaN included), and the next 16
+// are read while 16 are added. Measured on MI355X, one launch each:
+//   8 x 128 x 384:  pooling 8.0 -> 4.1 us, norm 6.2 -> 4.7 (one block per 256 columns and 8
+//                   loads before; one thread reading, squaring and adding)
+//   64 x 512 x 768: pooling 31 -> 15.6 us (6.4 TB/s), norm 15 -> 7.6
+constexpr int POOL_COLS = 64;
+
+__global__ __launch_bounds__(POOL_COLS) void pool_mean_cols(const float *__restrict__ h, int64_t ldh, int L, int D,
+                                                            float *__restrict__ out, int64_t ldo) {
+    const int j = blockIdx.x * POOL_COLS + threadIdx.x;
     if (j >= D) return;
     const float *col = h + (int64_t)blockIdx.y * L * ldh + j;
     double acc = 0.0;
     int i = 0;
-    for (; i + 8 <= L; i += 8) {  // 8 loads in flight, then the adds in row order
-        float x[8];
+    auto rows = [&](auto u_c, auto whole) {  // U loads in flight, then the adds in row order
+        constexpr int U = decltype(u_c)::value;
+        float x[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = col[(int64_t)(i + u) * ldh];
+        for (int u = 0; u < U; ++u) x[u] = col[(int64_t)(whole ? i + u : min(i + u, L - 1)) * ldh];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc += (double)x[u];
-    }
-    for (; i < L; ++i) acc += (double)col[(int64_t)i * ldh];
+        for (int u = 0; u < U; ++u)
+            if (whole || u < L - i) acc += (double)x[u];
+        i += min(U, L - i);
+    };
+    using Big = std::integral_constant<int, 32>;
+    using Small = std::integral_constant<int, 8>;
+    while (L - i >= 32) rows(Big{}, std::true_type{});
+    while (L - i >= 8) rows(Small{}, std::true_type{});
+    if (i < L) rows(Small{}, std::false_type{});
     out[blockIdx.y * ldo + j] = L > 0 ? (float)(acc * (1.0 / (double)L)) : 0.0f;
 }
 
 __global__ __launch_bounds__(256) void l2_normalize_rows(float *__restrict__ out, int64_t ldo, int D) {
-    __shared__ float row[4096];
+    constexpr int U = 16;
+    __shared__ __attribute__((aligned(16))) double sqs[4096 + U];
     __shared__ double norm_s;
     float *o = out + blockIdx.x * ldo;
-    for (int j = threadIdx.x; j < D; j += 256) row[j] = o[j];
+    const int padded = (D + U - 1) / U * U + U;  // the last read ahead included; D <= 4096
+    for (int j = threadIdx.x; j < padded; j += 256) {
+        const double x = j < D ? (double)o[j] : 0.0;
+        sqs[j] = x * x;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double sq = 0.0;
-        for (int j = 0; j < D; ++j) sq += (double)row[j] * (double)row[j];
+        double sq = 0.0, x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = sqs[u];
+        for (int j = 0; j < D; j += U) {
+            double y[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) y[u] = sqs[j + U + u];
+#pragma unroll
+            for (int u = 0; u < U; ++u) sq += x[u];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = y[u];
+        }
         norm_s = sqrt(sq);
     }
     __syncthreads();
