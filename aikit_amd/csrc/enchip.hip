@@ -621,6 +621,22 @@ void launch_skinny_topk(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq
     SK_SWITCH(nk)
 #undef SK_CASE
 }
+
+// The group maxima of M rows over the first `groups` 32-channel groups; aq is read up to a
+// multiple of 32 RB rows.
+template <int RB>
+void launch_skinny_maxima(const Weight &w, int nk, const int8_t *aq, const float *as, int64_t M, int64_t groups,
+                          uint64_t *maxima, hipStream_t s) {
+    using namespace enchip;
+    const dim3 grid((unsigned)(groups / SM_WAVES), (unsigned)((M + 32 * RB - 1) / (32 * RB))), block(64 * SM_WAVES);
+#define SK_CASE(NK)                                                                                             \
+    case NK:                                                                                                    \
+        hipLaunchKernelGGL((gemm_w8a8_skinny_maxima<RB, NK>), grid, block, 0, s, aq, w.d_w, as, w.d_s, (int)M,  \
+                           maxima);                                                                             \
+        break;
+    SK_SWITCH(nk)
+#undef SK_CASE
+}
 #undef SK_SWITCH
 
 // nk from skinny_nk; 32 x 4 or 32 x 8 rows staged.
@@ -2106,12 +2122,13 @@ int launch_topk(enchip_ctx *c, const float *scores, int64_t ld, int64_t rows, in
 
 // enchip_ann_topk's fused route: the selection runs in the scoring GEMM's epilogue, so the
 // M x N scores are never written or read back.
-//   1. gemm_w8a8_pt scores each row's first kSinkSample columns into d_dst, and stage 1
-//      + topk_thresh take the k-th largest key among them: a lower bound of the row's
-//      k-th largest key (the sample is part of the row). topk_thresh zeroes the counts.
-//   2. gemm_w8a8_pt<EPI_TOPK> scores every column and appends the scores whose key is at
-//      or above their row's bound to the row's list (gemm_persistent.h, TopkSink): the
-//      row's k largest keys are all there.
+//   1. A lower bound of each row's k-th largest key from its first kSinkSample columns, which
+//      also zeroes the counts: the k-th largest of the maxima of 32-column groups
+//      (gemm_w8a8_skinny_maxima, topk_thresh_maxima); where the skinny kernels don't take the
+//      shape, gemm_w8a8_pt's scores in d_dst, stage 1 and topk_thresh (the k-th largest of all).
+//   2. gemm_w8a8_skinny_topk or gemm_w8a8_pt<EPI_TOPK> scores every column and appends the
+//      scores whose key is at or above their row's bound to the row's list (gemm_persistent.h,
+//      TopkSink): the row's k largest keys are all there.
 //   3. topk_sink_merge selects the k largest of each list.
 // About k of every kSinkSample columns clear a bound on exchangeable scores (k * N /
 // kSinkSample per row); a row whose list overflows its capacity (sink_cap: adversarial
@@ -2144,23 +2161,38 @@ int launch_ann_fused(enchip_ctx *c, const Weight &w, int64_t M, int64_t k, hipSt
                      float *hit_s, unsigned *count) {
     using namespace enchip;
     int rc;
-    if ((rc = ensure(c, &c->d_dst, &c->dst_cap, (size_t)(M * kSinkSample) * sizeof(float)))) return rc;
-    const int64_t cand_n = M * TOPK_SAMPLE_CHUNKS * k, cap = sink_cap(k);
+    const int nk = skinny_shape_nk(w, c->d_aq, w.Kp, true);
+    if (!nk && (rc = ensure(c, &c->d_dst, &c->dst_cap, (size_t)(M * kSinkSample) * sizeof(float)))) return rc;
+    const int64_t cand_n = M * (nk ? TOPK_MAXIMA : TOPK_SAMPLE_CHUNKS * k), cap = sink_cap(k);
     const size_t words = (size_t)(cand_n + M + M * cap) + (size_t)(M * cap + 1) / 2;
     if ((rc = ensure(c, &c->d_cand, &c->cand_cap, words * sizeof(uint64_t)))) return rc;
     uint64_t *cand = c->d_cand, *thr = cand + cand_n, *keys = thr + M;
     float *raw = reinterpret_cast<float *>(keys + M * cap);
-    Weight sample = w;
-    sample.N = sample.Np = kSinkSample;
-    if ((rc = launch_gemm(c, sample, c->d_aq, w.Kp, c->d_as, nullptr, EPI_F32, c->d_dst, kSinkSample, M, s, true)))
-        return rc;
-    for (int64_t r0 = 0; r0 < M; r0 += 65535) {
-        const int64_t nr = std::min<int64_t>(65535, M - r0);
-        uint64_t *cr = cand + r0 * TOPK_SAMPLE_CHUNKS * k;
-        hipLaunchKernelGGL(topk_chunk_wide, dim3((unsigned)TOPK_SAMPLE_CHUNKS, (unsigned)nr), dim3(256), 0, s,
-                           c->d_dst + r0 * kSinkSample, kSinkSample, kSinkSample, (int)k, TOPK_SAMPLE_CHUNKS, cr, 0,
-                           (const uint64_t *)nullptr);
-        launch_thresh(cr, nr, TOPK_SAMPLE_CHUNKS, k, thr + r0, count + r0, s);
+    if (nk) {
+        const int64_t most = 64 * 65535;
+        for (int64_t r0 = 0; r0 < M; r0 += most) {
+            const int64_t mr = std::min(most, M - r0);
+            const int8_t *aq = c->d_aq + r0 * w.Kp;
+            const float *as = c->d_as + r0;
+            uint64_t *mx = cand + r0 * TOPK_MAXIMA;
+            if (mr <= 32) launch_skinny_maxima<1>(w, nk, aq, as, mr, TOPK_MAXIMA, mx, s);
+            else launch_skinny_maxima<2>(w, nk, aq, as, mr, TOPK_MAXIMA, mx, s);
+        }
+        hipLaunchKernelGGL(topk_thresh_maxima, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s, (const uint64_t *)cand, M,
+                           (int)k, thr, count);
+    } else {
+        Weight sample = w;
+        sample.N = sample.Np = kSinkSample;
+        if ((rc = launch_gemm(c, sample, c->d_aq, w.Kp, c->d_as, nullptr, EPI_F32, c->d_dst, kSinkSample, M, s, true)))
+            return rc;
+        for (int64_t r0 = 0; r0 < M; r0 += 65535) {
+            const int64_t nr = std::min<int64_t>(65535, M - r0);
+            uint64_t *cr = cand + r0 * TOPK_SAMPLE_CHUNKS * k;
+            hipLaunchKernelGGL(topk_chunk_wide, dim3((unsigned)TOPK_SAMPLE_CHUNKS, (unsigned)nr), dim3(256), 0, s,
+                               c->d_dst + r0 * kSinkSample, kSinkSample, kSinkSample, (int)k, TOPK_SAMPLE_CHUNKS, cr, 0,
+                               (const uint64_t *)nullptr);
+            launch_thresh(cr, nr, TOPK_SAMPLE_CHUNKS, k, thr + r0, count + r0, s);
+        }
     }
     if ((rc = check_launch(c, "ann_topk sample"))) return rc;
     TopkSink sink;
@@ -2169,7 +2201,7 @@ int launch_ann_fused(enchip_ctx *c, const Weight &w, int64_t M, int64_t k, hipSt
     sink.key = keys;
     sink.score = raw;
     sink.cap = (int)cap;
-    if (const int nk = skinny_shape_nk(w, c->d_aq, w.Kp, true)) {
+    if (nk) {
         // 256 rows a launch (each reads the index once) while a row lists in one workgroup, as
         // expected, half of its LDS slots there or less (k N / kSinkSample / workgroups); past
         // that every other candidate would go to the global lists one by one. Measured on MI355X

@@ -594,6 +594,47 @@ __global__ __launch_bounds__(256) void topk_thresh_sorted(const uint64_t *__rest
     }
 }
 
+// The row thresholds from the maxima of TOPK_MAXIMA groups of a row's scores (keys, 0 for a group
+// of NaN): the k-th largest of them, or 0 when fewer than k are nonzero. One wavefront per row
+// searches it bit by bit, counting by ballot, and stops at a value that exactly k keys reach.
+constexpr int TOPK_MAXIMA = TOPK_SAMPLE_CHUNKS * TOPK_WCHUNK / 32;
+
+__global__ __launch_bounds__(256) void topk_thresh_maxima(const uint64_t *__restrict__ maxima, int64_t rows, int k,
+                                                          uint64_t *__restrict__ thr, unsigned *__restrict__ zero) {
+    constexpr int PER_LANE = TOPK_MAXIMA / 64;
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    uint64_t v[PER_LANE];
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) v[i] = maxima[row * TOPK_MAXIMA + lane + 64 * i];
+    uint64_t t = 0;  // at least k keys are >= t, once it is not 0
+    int n = 0;
+    for (int bit = 31; bit >= 0 && n != k; --bit) {  // the scores' bits
+        const uint32_t c = (uint32_t)(t >> 32) | 1u << bit;
+        n = 0;
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i)
+            n += __builtin_popcountll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) >= c));
+        if (n >= k) t = (uint64_t)c << 32;
+    }
+    for (int bit = 31; bit >= 0 && n != k && t != 0; --bit) {  // more than k reach it: the indices'
+        const uint64_t c = t | 1u << bit;
+        n = 0;
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[i] >= c));
+        if (n >= k) t = c;
+    }
+    uint64_t low = 0;  // the complement of the smallest key >= t: the k-th largest
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) low = v[i] >= t && ~v[i] > low ? ~v[i] : low;
+    low = wave_max_u64(low);
+    if (lane == 0) {
+        thr[row] = t == 0 ? 0 : ~low;
+        zero[row] = 0;  // the row's TopkSink count
+    }
+}
+
 // The merge after the fused scoring GEMM (gemm_w8a8_pt<EPI_TOPK>): one workgroup per row
 // takes the k largest (k <= KMAX) of the count[row] candidates the GEMM kept (keys at
 // key[row*cap ..], their scores at score[row*cap ..], unordered), and writes indices and
