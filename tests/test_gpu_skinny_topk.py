@@ -49,3 +49,32 @@ def test_candidates_match_oracle(ctx, M, N, K, k, odd):
         assert hi[r, :idx.size].tolist() == idx.tolist(), f"row {r}: indices differ"
         assert np.array_equal(hs[r, :idx.size].view(np.uint32), sc.view(np.uint32)), f"row {r}: scores differ"
         assert (hi[r, idx.size:] == -1).all() and np.isnan(hs[r, idx.size:]).all(), f"row {r}: padding"
+
+
+@pytest.mark.parametrize("k,live", [(10, 10), (10, 9), (64, 1024)])
+def test_bounds_of_few_live_groups(ctx, k, live):
+    # NaN index scales leave `live` of the sample's 1024 column groups a score: the k-th largest
+    # group maximum, or no bound where fewer than k have one (every score is listed, the lists
+    # overflow and the two-pass route answers). Equal codes, so ties go by index.
+    M, N, K = 40, 131072, 128
+    g = workloads.rng(7900 + k + live)
+    q = np.abs(workloads.activations(g, M, K)) + np.float32(0.01)
+    codes = np.ones((N, K), np.int8)
+    scales = np.full(N, 1e-3, np.float32)
+    sample = np.full((1024, 32), np.nan, np.float32)
+    sample[g.permutation(1024)[:live], g.integers(0, 32)] = 2e-3
+    scales[:32768] = sample.reshape(-1)
+    print(f"[case] skinny bounds k={k} live={live}", flush=True)
+    w = ctx.register_weight(codes, scales)
+    try:
+        _, b0 = ctx.ann_topk_stats()
+        hi, hs = ctx.ann_topk(w, q, k)
+        _, b1 = ctx.ann_topk_stats()
+    finally:
+        ctx.release_weight(w)
+    assert b1 - b0 == (1 if live < k else 0), "route"
+    scores = oracle.w8a8_linear(q, codes, scales, None, 0, M, K, N)
+    for r in range(M):
+        idx, sc = oracle.top_hits(scores[r], k)
+        assert hi[r].tolist() == idx.tolist(), f"row {r}: indices differ"
+        assert np.array_equal(hs[r].view(np.uint32), sc.view(np.uint32)), f"row {r}: scores differ"
