@@ -21,9 +21,9 @@
 // times the other operand.) The contract is the reference's gate against a float64 dot
 // product (gpu/enccuda/backend_test.go:47-86).
 // An operand the split cannot hold (an infinity, or a value that rounds to one in bf16) or a
-// sum that overflows leaves a non-finite accumulator; the 32 x 32 blocks of a wavefront that
-// sees one are computed again by f32_block on the f32 MFMA, so infinities and overflow give
-// what f32 arithmetic gives.
+// sum that overflows leaves a non-finite output; those are computed again by f32_block on the f32
+// MFMA, so infinities and overflow give what f32 arithmetic gives. The other outputs of the block
+// keep their split sums.
 //
 // bf16 products run at 16 times the f32 MFMA's rate, so the six cost 0.38 of it; the f32
 // kernel these replace reached 110-120 of its 154 TFLOP/s at 4096^2 and less than a third of
@@ -98,8 +98,9 @@ __device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN]) {
     return s != 0.0f;  // 0, or NaN
 }
 
-// The 32 x 32 outputs at (m0, n0) of one wavefront on the f32 MFMA, operands loaded value by
-// value: for the rare blocks whose split sums are not finite.
+// The 32 x 32 outputs at (m0, n0), stored from split sums, computed by one wavefront on the f32
+// MFMA with operands loaded value by value, and stored where the split sum is not finite: the others
+// keep theirs, whatever the tile.
 template <bool BKN>
 __device__ __forceinline__ void f32_block(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc,
                                        int M, int N, int K, int m0, int n0) {
@@ -122,7 +123,9 @@ __device__ __forceinline__ void f32_block(const float *A, int64_t lda, const flo
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
         const int row = m0 + acc_row(e, lane);
-        if (row < M) C[(int64_t)row * ldc + n0 + r] = acc[e];
+        if (row >= M) continue;
+        float *c = C + (int64_t)row * ldc + n0 + r;
+        if (!(fabsf(*c) < INFINITY)) *c = acc[e];
     }
 }
 
@@ -282,12 +285,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
         for (int s = 0; s < KC / 16; ++s) mfma_parts<TM, TN>(pa[s], pb[s], acc);
         lds_barrier();
     }
+    const bool nonfinite = __builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc)) != 0;
     const int m0 = bm0 + 32 * TM * wm, n0 = bn0 + 32 * TN * wn;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc)) != 0, 0)) {
-        for (int u = 0; u < TM * TN; ++u)
-            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -300,6 +299,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
                 if (row < M) C[(int64_t)row * ldc + col] = acc[i][t][e];
             }
         }
+    if (__builtin_expect(nonfinite, 0))
+        for (int u = 0; u < TM * TN; ++u)
+            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
 }
 
 // K split: 4 wavefronts per (32 TM) x (32 TN) tile, wavefront w taking the 32-deep chunks w, w +
@@ -404,11 +406,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
             }
         }
     }
-    if (__builtin_expect(__syncthreads_or(any_nonfinite<TM, TN>(acc)), 0)) {
-        for (int u = wave; u < TM * TN; u += WK)
-            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -429,17 +426,20 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
             const f32x4 o = *reinterpret_cast<const f32x4 *>(&red[w][at]);
             v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
         }
+        const float x[4] = {v.x, v.y, v.z, v.w};
         if (row >= M) continue;
         float *o = C + (int64_t)row * ldc + col;
         if (vst) {
             if (col < N) *reinterpret_cast<f32x4 *>(o) = v;
         } else {
-            const float x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int u = 0; u < 4; ++u)
                 if (col + u < N) o[u] = x[u];
         }
     }
+    if (__builtin_expect(__syncthreads_or(any_nonfinite<TM, TN>(acc)), 0))
+        for (int u = wave; u < TM * TN; u += WK)
+            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
 }
 
 // C = 0 for a K = 0 product (the empty dot product), grid (ceil(M*N/256), inner, outer).

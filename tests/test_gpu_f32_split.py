@@ -89,3 +89,45 @@ def test_a_batch_gives_each_problem_its_own_bits(ctx):
             ctx.matmul_bt_f32_dev(a[i].data_ptr(), K, b[i].data_ptr(), K, enchip.B_NK, c2[i].data_ptr(), N, M, K, N)
         torch.cuda.synchronize()
         assert torch.equal(c1.view(torch.int32), c2.view(torch.int32))
+
+
+def product(ctx, a, b, layout):
+    """a[M, K] . b[N, K]^T from device buffers, B in either layout."""
+    import torch
+
+    (M, K), N = a.shape, b.shape[0]
+    da = torch.from_numpy(a).cuda()
+    db = torch.from_numpy(np.ascontiguousarray(b if layout == enchip.B_NK else b.T)).cuda()
+    dc = torch.full((M, N), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.matmul_bt_f32_dev(da.data_ptr(), K, db.data_ptr(), K if layout == enchip.B_NK else N, layout, dc.data_ptr(), N,
+                          M, K, N)
+    torch.cuda.synchronize()
+    return dc.cpu().numpy()
+
+
+@pytest.mark.parametrize("M,K,N", [(130, 300, 200), (40, 512, 160), (300, 64, 300), (65, 40, 100), (1200, 96, 1500)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 3.4e38])
+def test_outputs_beside_a_special_value_keep_their_bits(ctx, M, K, N, bad):
+    # one row of A and one of B hold a value the split cannot: every other output has the bits of
+    # the product without them, in one problem and in a batch of 24 (other tile sizes)
+    import torch
+
+    g = workloads.rng(6500 + M)
+    a, b = g.standard_normal((M, K)).astype(np.float32), g.standard_normal((N, K)).astype(np.float32)
+    print(f"[case] f32 beside {bad} M={M} K={K} N={N}", flush=True)
+    clean = product(ctx, a, b, enchip.B_NK)
+    i, j = M // 2, N // 3
+    a[i, K // 2], b[j, 1] = bad, bad
+    with np.errstate(all="ignore"):
+        one = product(ctx, a, b, enchip.B_NK)
+    keep = np.ones((M, N), bool)
+    keep[i], keep[:, j] = False, False
+    assert np.array_equal(one.view(np.int32)[keep], clean.view(np.int32)[keep])
+    da, db = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    dc = torch.empty((24, M, N), device="cuda")
+    torch.cuda.synchronize()
+    ctx.matmul_bt_f32_dev(da.data_ptr(), K, db.data_ptr(), K, enchip.B_NK, dc.data_ptr(), N, M, K, N,
+                          inner=(24, 0, 0, M * N))
+    torch.cuda.synchronize()
+    assert np.array_equal(dc.cpu().numpy().view(np.int32), np.broadcast_to(one.view(np.int32), (24, M, N)))
