@@ -417,6 +417,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
     static_assert(BM * RL % NT == 0, "whole passes");
     const int c4 = 4 * (tid % RL), r0 = tid / RL, col = n0 + c4;
     const bool vst = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C & 15) == 0;
+    float zeros = 0.0f;  // NaN where a sum is not finite
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         const int at = (r0 + RP * g) * P + c4, row = m0 + r0 + RP * g;
@@ -427,6 +428,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
             v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
         }
         const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) zeros += x[u] * 0.0f;
         if (row >= M) continue;
         float *o = C + (int64_t)row * ldc + col;
         if (vst) {
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
                 if (col + u < N) o[u] = x[u];
         }
     }
-    if (__builtin_expect(__syncthreads_or(any_nonfinite<TM, TN>(acc)), 0))
+    if (__builtin_expect(__syncthreads_or(zeros != 0.0f), 0))
         for (int u = wave; u < TM * TN; u += WK)
             f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
 }

@@ -131,3 +131,17 @@ def test_outputs_beside_a_special_value_keep_their_bits(ctx, M, K, N, bad):
                           inner=(24, 0, 0, M * N))
     torch.cuda.synchronize()
     assert np.array_equal(dc.cpu().numpy().view(np.int32), np.broadcast_to(one.view(np.int32), (24, M, N)))
+
+
+@pytest.mark.parametrize("N", [256, 1031])
+@pytest.mark.parametrize("layout", [enchip.B_NK, enchip.B_KN])
+def test_partial_sums_that_overflow_together(ctx, N, layout):
+    # K split over wavefronts: in 32-deep chunks 0, 2 and 5 (wavefronts 0, 2 and 1) 2e38, -2e38 and
+    # 2e38. Adding the wavefronts' sums in their order overflows; f32 adds in k order do not.
+    a = np.zeros((33, 1024), np.float32)
+    a[::2, 0], a[::2, 64], a[::2, 160] = 2e38, -2e38, 2e38
+    a[1::2] = np.float32(0.25)
+    b = np.ones((N, 1024), np.float32)
+    print(f"[case] f32 partial sums N={N} layout={layout}", flush=True)
+    got = product(ctx, a, b, layout)
+    assert (got[::2] == np.float32(2e38)).all() and (got[1::2] == 256).all()
