@@ -9,7 +9,7 @@
 // B is [N, K] rows (MatmulBT's b, BKN = false) or [K, N] rows (BKN = true: V itself
 // for scores . V, element (n, k) at B[k*ldb + n], so no transpose copy either).
 //
-// Arithmetic. Every operand value is split exactly into three bf16 parts, x = h + m + l (h
+// Arithmetic. Every operand value is split into three bf16 parts, x = h + m + l (h
 // the bf16 nearest x, m the one nearest x - h, l the rest, which has at most 8 bits), and a
 // product is the six products of parts above 2^-25 of it: h.h', h.m', m.h', m.m', h.l', l.h',
 // each exact on v_mfma_f32_32x32x16_bf16 and summed in f32. The three left out, m.l', l.m'
@@ -17,9 +17,13 @@
 // 16-deep step rounds the sum 6 times where the f32 MFMA (32x32x2) rounds it 8 to 16 times.
 // Measured against float64 (standard normal operands, relative 2-norm): K = 768 4.2e-7, or
 // 2.1e-7 with K split over wavefronts, against the f32 MFMA's 5.0e-7; K = 3072 8.7e-7 /
-// 4.3e-7 against 9.9e-7. (Parts below 2^-126 may be flushed: an absolute error under 2^-126
-// times the other operand.) The contract is the reference's gate against a float64 dot
-// product (gpu/enccuda/backend_test.go:47-86).
+// 4.3e-7 against 9.9e-7. The contract is the reference's gate against a float64 dot product
+// (gpu/enccuda/backend_test.go:47-86).
+// The split is exact for operands from 2^-110 up (bf16 subnormals are kept, in the conversions and
+// in the MFMA). Outputs that can have lost by smaller ones are computed again on the f32 MFMA (see
+// kBelow): with |a| near 2^-120 and |b| near 2^120 the worst relative error was 1.1e-5 without,
+// 3.9e-7 with, as on the f32 MFMA throughout. The looking costs up to 3%: 4096 x 768, K = 768 40.0 ->
+// 41.3 us, 512 x 3072 25.4 -> 26.0, 4096 x 3072, K = 3072 391 -> 395, K-split shapes none.
 // An operand the split cannot hold (an infinity, or a value that rounds to one in bf16) or a
 // sum that overflows leaves a non-finite output; those are computed again by f32_block on the f32
 // MFMA, so infinities and overflow give what f32 arithmetic gives. The other outputs of the block
@@ -63,8 +67,10 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The three bf16 parts of a (low half) and b (high half of each word).
-__device__ __forceinline__ void split3_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+// The three bf16 parts of a (low half) and b (high half of each word); big: the largest magnitude
+// so far.
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l, float &big) {
+    big = fmaxf(fmaxf(fabsf(a), fabsf(b)), big);  // one v_max3
     h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
     const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
     m = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
@@ -85,22 +91,55 @@ __device__ __forceinline__ void mfma_parts(const bf16x8 (&pa)[TM][3], const bf16
                 acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][pi[u]], pb[t][qi[u]], acc[i][t], 0, 0, 0);
 }
 
-// Whether any accumulator of the lane is infinite or NaN.
+// Where the parts are not the operand. bf16's last bit is 2^-133, so a nonzero operand under
+// 2^-110 (kBelow, of the word below_split gives; zeros give the largest) may lose up to 2^-134. A
+// sum of K products with every operand at most kBig then lost at most 2 K 2^-134 kBig = K 2^-109,
+// under 2^-25 of any output from lost_below(K) up. So the main loop only looks for operands above
+// kBig, and the end for outputs below that (zeros, as a rule): blocks with either have their
+// operands searched for small ones, and f32_block computes the outputs that can have lost by it.
+// (Looking for the small ones in the main loop cost up to 12%.)
+constexpr uint32_t kBelow = ((127u - 110u) << 24) - 1u;
+constexpr float kBig = 0x1p24f;
+__device__ __forceinline__ uint32_t below_split(float x) { return (__float_as_uint(x) << 1) - 1u; }
+__device__ __forceinline__ float lost_below(int K) { return (float)K * 0x1p-84f; }
+
+// Whether any of the lane's outputs is infinite or NaN, and their smallest magnitude.
 template <int TM, int TN>
-__device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN]) {
+__device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN], float &least) {
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int t = 0; t < TN; ++t)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s += acc[i][t][e] * 0.0f;
+            for (int e = 0; e < 16; ++e) {
+                s += acc[i][t][e] * 0.0f;
+                least = fminf(fabsf(acc[i][t][e]), least);
+            }
     return s != 0.0f;  // 0, or NaN
 }
 
+// Whether a nonzero value under 2^-110 is among the `rows` rows at p (pitch ld, n values each), by
+// one wavefront.
+__device__ __forceinline__ bool holds_small(const float *p, int64_t ld, int rows, int n) {
+    uint32_t low = ~0u;
+    for (int i = 0; i < rows; ++i)
+        for (int k = threadIdx.x & 63; k < n; k += 64) low = min(low, below_split(p[i * ld + k]));
+    return __builtin_amdgcn_ballot_w64(low < kBelow) != 0;
+}
+
+template <bool BKN>
+__device__ __forceinline__ bool operands_small(const float *A, int64_t lda, const float *B, int64_t ldb, int M, int N, int K,
+                                            int m0, int n0, int rows, int cols) {
+    const int m = min(rows, M - m0), n = min(cols, N - n0);
+    if (m <= 0 || n <= 0) return false;
+    return holds_small(A + (int64_t)m0 * lda, lda, m, K) ||
+           (BKN ? holds_small(B + n0, ldb, K, n) : holds_small(B + (int64_t)n0 * ldb, ldb, n, K));
+}
+
 // The 32 x 32 outputs at (m0, n0), stored from split sums, computed by one wavefront on the f32
-// MFMA with operands loaded value by value, and stored where the split sum is not finite: the others
-// keep theirs, whatever the tile.
+// MFMA with operands loaded value by value, and stored where the split sum is not finite or can have
+// lost by a small operand: whatever the tile, each output by its own row, column and split sum.
 template <bool BKN>
 __device__ __forceinline__ void f32_block(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc,
                                        int M, int N, int K, int m0, int n0) {
@@ -111,21 +150,32 @@ __device__ __forceinline__ void f32_block(const float *A, int64_t lda, const flo
     f32x16 acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    float big_a = 0.0f, big_b = 0.0f;  // of row m0 + r, of column n0 + r
+    uint32_t low_a = ~0u, low_b = ~0u;
     for (int k0 = 0; k0 < K; k0 += 16) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             const int k = k0 + kh + s, kc = min(k, K - 1);
-            const float a = pa[kc], b = BKN ? B[(int64_t)kc * ldb + n] : B[(int64_t)n * ldb + kc];
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < K ? a : 0.0f, k < K ? b : 0.0f, acc, 0, 0, 0);
+            const float av = pa[kc], bv = BKN ? B[(int64_t)kc * ldb + n] : B[(int64_t)n * ldb + kc];
+            const float a = k < K ? av : 0.0f, b = k < K ? bv : 0.0f;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+            big_a = fmaxf(big_a, fabsf(a)), big_b = fmaxf(big_b, fabsf(b));
+            low_a = min(low_a, below_split(a)), low_b = min(low_b, below_split(b));
         }
     }
-    if (n0 + r >= N) return;
+    big_a = fmaxf(big_a, __shfl_xor(big_a, 32)), big_b = fmaxf(big_b, __shfl_xor(big_b, 32));
+    low_a = min(low_a, (uint32_t)__shfl_xor((int)low_a, 32)), low_b = min(low_b, (uint32_t)__shfl_xor((int)low_b, 32));
+    const float small_out = lost_below(K);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-        const int row = m0 + acc_row(e, lane);
-        if (row >= M) continue;
+        const int at = acc_row(e, lane), row = m0 + at;
+        const float ba = __shfl(big_a, at);
+        const uint32_t la = (uint32_t)__shfl((int)low_a, at);
+        if (row >= M || n0 + r >= N) continue;
         float *c = C + (int64_t)row * ldc + n0 + r;
-        if (!(fabsf(*c) < INFINITY)) *c = acc[e];
+        const float old = *c;
+        const bool lost = min(la, low_b) < kBelow && (fabsf(old) < small_out || fmaxf(ba, big_b) > kBig);
+        if (lost || !(fabsf(old) < INFINITY)) *c = acc[e];
     }
 }
 
@@ -154,7 +204,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
     static_assert(AV >= 1 && BV >= 1 && (KNI % NT == 0 || KNI < NT) && STAGE * 2 <= 128 * 1024, "tile");
     const bool kn_mine = KNI >= NT || (int)threadIdx.x < KNI;
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+    __shared__ int any_big;  // the block has an operand above kBig
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
+    if (tid == 0) any_big = 0;
     const int64_t y = blockIdx.y, z = blockIdx.z;
     A += y * s1.a + z * s2.a;
     B += y * s1.b + z * s2.b;
@@ -180,6 +232,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
         else gb[i] = B + (int64_t)min(bn0 + lr + (NT / LPR) * i, N - 1) * ldb;
     }
     f32x4 ra[AV], rb[BV];
+    float big = 0.0f;
     auto load_row = [&](const float *p, int k) -> f32x4 {
         if (VEC) return *reinterpret_cast<const f32x4 *>(p + min(k, K - 4));
         return f32x4{p[min(k, K - 1)], p[min(k + 1, K - 1)], p[min(k + 2, K - 1)], p[min(k + 3, K - 1)]};
@@ -214,8 +267,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
             v.x = k < K ? v.x : 0.f, v.y = k + 1 < K ? v.y : 0.f, v.z = k + 2 < K ? v.z : 0.f, v.w = k + 3 < K ? v.w : 0.f;
         }
         uint32_t h0, m0, l0, h1, m1, l1;
-        split3_pair(v.x, v.y, h0, m0, l0);
-        split3_pair(v.z, v.w, h1, m1, l1);
+        split3_pair(v.x, v.y, h0, m0, l0, big);
+        split3_pair(v.z, v.w, h1, m1, l1, big);
         char *d = plane + row * P + 2 * lk;
         *reinterpret_cast<uint2 *>(d) = make_uint2(h0, h1);
         *reinterpret_cast<uint2 *>(d + stride) = make_uint2(m0, m1);
@@ -237,7 +290,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     uint32_t h, m, l;
-                    split3_pair(uu[e], ww[e], h, m, l);
+                    split3_pair(uu[e], ww[e], h, m, l, big);
                     char *d = bp + (4 * pg(i) + e) * P + 4 * pk;
                     *reinterpret_cast<uint32_t *>(d) = h;
                     *reinterpret_cast<uint32_t *>(d + PLB) = m;
@@ -285,7 +338,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
         for (int s = 0; s < KC / 16; ++s) mfma_parts<TM, TN>(pa[s], pb[s], acc);
         lds_barrier();
     }
-    const bool nonfinite = __builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc)) != 0;
+    if (big > kBig) any_big = 1;
+    lds_barrier();
+    float least = INFINITY;
+    const bool nonfinite = __builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc, least)) != 0;
+    const bool doubt = any_big != 0 || __builtin_amdgcn_ballot_w64(least < lost_below(K)) != 0;
     const int m0 = bm0 + 32 * TM * wm, n0 = bn0 + 32 * TN * wn;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -299,9 +356,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
                 if (row < M) C[(int64_t)row * ldc + col] = acc[i][t][e];
             }
         }
-    if (__builtin_expect(nonfinite, 0))
-        for (int u = 0; u < TM * TN; ++u)
-            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+    if (__builtin_expect(nonfinite || doubt, 0)) {
+        if (nonfinite || operands_small<BKN>(A, lda, B, ldb, M, N, K, m0, n0, 32 * TM, 32 * TN))
+            for (int u = 0; u < TM * TN; ++u)
+                f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+    }
 }
 
 // K split: 4 wavefronts per (32 TM) x (32 TN) tile, wavefront w taking the 32-deep chunks w, w +
@@ -336,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
         const int n = min(n0 + 32 * t + r, N - 1);
         pb[t] = BKN ? B + n : B + (int64_t)n * ldb;
     }
-    float ra[2][TM][8], rb[2][TN][8];
+    float ra[2][TM][8], rb[2][TN][8], big = 0.0f;
     auto load_row = [&](const float *p, int k, float (&v)[8]) {
         if (VEC) {
 #pragma unroll
@@ -366,7 +425,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
     auto split8 = [&](const float (&x)[8], bf16x8 (&p)[3]) {
         uint32_t h[4], m[4], l[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) split3_pair(x[2 * i], x[2 * i + 1], h[i], m[i], l[i]);
+        for (int i = 0; i < 4; ++i) split3_pair(x[2 * i], x[2 * i + 1], h[i], m[i], l[i], big);
         p[0] = __builtin_bit_cast(bf16x8, (u32x4{h[0], h[1], h[2], h[3]}));
         p[1] = __builtin_bit_cast(bf16x8, (u32x4{m[0], m[1], m[2], m[3]}));
         p[2] = __builtin_bit_cast(bf16x8, (u32x4{l[0], l[1], l[2], l[3]}));
@@ -417,7 +476,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
     static_assert(BM * RL % NT == 0, "whole passes");
     const int c4 = 4 * (tid % RL), r0 = tid / RL, col = n0 + c4;
     const bool vst = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C & 15) == 0;
-    float zeros = 0.0f;  // NaN where a sum is not finite
+    float zeros = 0.0f, least = INFINITY;  // of the sums: NaN where one is not finite; the smallest
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         const int at = (r0 + RP * g) * P + c4, row = m0 + r0 + RP * g;
@@ -429,7 +488,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
         }
         const float x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int u = 0; u < 4; ++u) zeros += x[u] * 0.0f;
+        for (int u = 0; u < 4; ++u) {
+            zeros += x[u] * 0.0f;
+            least = fminf(fabsf(x[u]), least);
+        }
         if (row >= M) continue;
         float *o = C + (int64_t)row * ldc + col;
         if (vst) {
@@ -440,9 +502,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
                 if (col + u < N) o[u] = x[u];
         }
     }
-    if (__builtin_expect(__syncthreads_or(zeros != 0.0f), 0))
-        for (int u = wave; u < TM * TN; u += WK)
-            f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+    const bool nonfinite = zeros != 0.0f;
+    if (__builtin_expect(__syncthreads_or(nonfinite || big > kBig || least < lost_below(K)), 0)) {
+        const bool redo = __syncthreads_or(nonfinite);
+        for (int u = wave; u < TM * TN; u += WK) {
+            const int mu = m0 + 32 * (u / TN), nu = n0 + 32 * (u % TN);
+            if (redo || operands_small<BKN>(A, lda, B, ldb, M, N, K, mu, nu, 32, 32))
+                f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, mu, nu);
+        }
+    }
 }
 
 // C = 0 for a K = 0 product (the empty dot product), grid (ceil(M*N/256), inner, outer).

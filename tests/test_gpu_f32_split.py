@@ -145,3 +145,63 @@ def test_partial_sums_that_overflow_together(ctx, N, layout):
     print(f"[case] f32 partial sums N={N} layout={layout}", flush=True)
     got = product(ctx, a, b, layout)
     assert (got[::2] == np.float32(2e38)).all() and (got[1::2] == 256).all()
+
+
+# the K split in each tile size, then the tile forms; K and N multiples of 4 or not
+@pytest.mark.parametrize("M,K,N", [(33, 300, 132), (500, 257, 1000), (130, 1024, 1031), (70, 40, 100), (500, 200, 2050),
+                                   (1200, 96, 1500), (1999, 31, 2301)])
+@pytest.mark.parametrize("layout", [enchip.B_NK, enchip.B_KN])
+@pytest.mark.parametrize("ea,eb,where", [(-112, 110, "all"), (-120, 118, "all"), (-127, 120, "all"), (-140, 124, "few"),
+                                         (118, -120, "all"), (120, -126, "few")])
+def test_small_operands_keep_f32_precision(ctx, M, K, N, layout, ea, eb, where):
+    # Operands near 2^ea and 2^eb, the small ones (f32 subnormals among them) too small for three
+    # bf16 parts: everywhere, or a few of them among zeros and values of ordinary size. One
+    # rounded add per product, and a product's rounding: (K + 2) 2^-24 sum |a b|, and 2^-149 a
+    # product where it is subnormal.
+    g = workloads.rng(6100 + M + ea)
+    a = (1 + g.random((M, K))).astype(np.float32) * g.choice(np.float32([-1, 1]), size=(M, K))
+    b = (1 + g.random((N, K))).astype(np.float32)
+    small, big, es, eg = (a, b, ea, eb) if ea < eb else (b, a, eb, ea)
+    if where == "all":
+        small[:] = np.ldexp(small, es)
+        big[:] = np.ldexp(big, eg)
+    else:
+        few = g.random(small.shape) < 2.0 / K
+        few[: small.shape[0] // 2] = False
+        small[:] = np.where(few, np.ldexp(small, es), np.where(g.random(small.shape) < 0.5, 0, small))
+        big[:, :] = np.where(g.random(big.shape) < 0.5, np.ldexp(big, eg - 20), np.ldexp(big, -100))
+    print(f"[case] f32 small operands M={M} K={K} N={N} layout={layout} 2^{ea} 2^{eb} {where}", flush=True)
+    got = product(ctx, a, b, layout)
+    ref = a.astype(np.float64) @ b.astype(np.float64).T
+    lim = (K + 2) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T) + K * 2.0**-149
+    assert np.all(np.abs(got - ref) <= lim)
+
+
+@pytest.mark.parametrize("M,K,N", [(96, 512, 160), (300, 64, 300), (40, 24, 2500)])
+def test_small_operands_beside_others_in_any_tile(ctx, M, K, N):
+    # 24 problems in a launch and one by one (other tile sizes): small operands in a few rows of A
+    # and of B, zero rows beside them, one value above 2^24: the same bits for every output.
+    import torch
+
+    g = workloads.rng(6900 + M)
+    a = g.standard_normal((24, M, K)).astype(np.float32)
+    b = g.standard_normal((24, N, K)).astype(np.float32)
+    for p in range(24):
+        a[p, g.integers(0, M, 3)] = 0
+        a[p, g.integers(0, M, 3), g.integers(0, K, 3)] = np.float32(2.0**-125 * 1.7)
+        a[p, g.integers(0, M)] *= np.float32(2.0**-115)
+        b[p, g.integers(0, N), g.integers(0, K)] = np.float32(2.0**100 if p % 2 else -(2.0**-149))
+    da, db = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    c1, c2 = torch.empty((24, M, N), device="cuda"), torch.empty((24, M, N), device="cuda")
+    torch.cuda.synchronize()
+    print(f"[case] f32 small operands, batch of 24 M={M} K={K} N={N}", flush=True)
+    ctx.matmul_bt_f32_dev(da.data_ptr(), K, db.data_ptr(), K, enchip.B_NK, c1.data_ptr(), N, M, K, N,
+                          inner=(24, M * K, N * K, M * N))
+    for i in range(24):
+        ctx.matmul_bt_f32_dev(da[i].data_ptr(), K, db[i].data_ptr(), K, enchip.B_NK, c2[i].data_ptr(), N, M, K, N)
+    torch.cuda.synchronize()
+    assert torch.equal(c1.view(torch.int32), c2.view(torch.int32))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    ref = np.matmul(a64, b64.transpose(0, 2, 1))
+    lim = (6 * -(-K // 16) + 6 + K) * 2.0**-24 * np.matmul(np.abs(a64), np.abs(b64).transpose(0, 2, 1)) + K * 2.0**-149
+    assert np.all(np.abs(c1.cpu().numpy() - ref) <= lim)
