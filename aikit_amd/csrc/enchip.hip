@@ -622,17 +622,17 @@ void launch_skinny_topk(enchip_ctx *c, const Weight &w, int nk, const int8_t *aq
 #undef SK_CASE
 }
 
-// The group maxima of M rows over the first `groups` 32-channel groups; aq is read up to a
-// multiple of 32 RB rows.
+// The sample's group maxima of M rows, in maxima_parts(M) parts; aq is read up to a multiple of 32
+// RB rows.
 template <int RB>
-void launch_skinny_maxima(const Weight &w, int nk, const int8_t *aq, const float *as, int64_t M, int64_t groups,
+void launch_skinny_maxima(const Weight &w, int nk, const int8_t *aq, const float *as, int64_t M, int64_t parts,
                           uint64_t *maxima, hipStream_t s) {
     using namespace enchip;
-    const dim3 grid((unsigned)(groups / SM_WAVES), (unsigned)((M + 32 * RB - 1) / (32 * RB))), block(64 * SM_WAVES);
+    const dim3 grid((unsigned)(32 * parts), (unsigned)((M + 32 * RB - 1) / (32 * RB))), block(64 * SM_WAVES);
 #define SK_CASE(NK)                                                                                             \
     case NK:                                                                                                    \
         hipLaunchKernelGGL((gemm_w8a8_skinny_maxima<RB, NK>), grid, block, 0, s, aq, w.d_w, as, w.d_s, (int)M,  \
-                           maxima);                                                                             \
+                           (int)parts, maxima);                                                                 \
         break;
     SK_SWITCH(nk)
 #undef SK_CASE
@@ -2123,7 +2123,7 @@ int launch_topk(enchip_ctx *c, const float *scores, int64_t ld, int64_t rows, in
 // enchip_ann_topk's fused route: the selection runs in the scoring GEMM's epilogue, so the
 // M x N scores are never written or read back.
 //   1. A lower bound of each row's k-th largest key from its first kSinkSample columns, which
-//      also zeroes the counts: the k-th largest of the maxima of 32-column groups
+//      also zeroes the counts: the k-th largest of the maxima of 1024 groups of 32 columns
 //      (gemm_w8a8_skinny_maxima, topk_thresh_maxima); where the skinny kernels don't take the
 //      shape, gemm_w8a8_pt's scores in d_dst, stage 1 and topk_thresh (the k-th largest of all).
 //   2. gemm_w8a8_skinny_topk or gemm_w8a8_pt<EPI_TOPK> scores every column and appends the
@@ -2154,6 +2154,15 @@ bool ann_fused_ok(const enchip_ctx *c, const Weight &w, int64_t M, int64_t k, bo
                   use_persistent(w, nullptr, w.Kp, nullptr, w.N, M, true));
 }
 
+// Workgroups that share one group of the sample's maxima (gemm_w8a8_skinny_maxima): enough for one
+// workgroup per CU. Each more costs topk_thresh_maxima loads: on MI355X, maxima + bounds for K = 384
+// in 1, 2 and 4 parts: 64 rows 26.1, 20.3, 17.6 us, 256 rows 27.3, 22.4, 24.3, 1024 rows 41.0, 44.4,
+// 49.7.
+int64_t maxima_parts(const enchip_ctx *c, int64_t M) {
+    const int64_t blocks = 32 * ((M + 63) / 64);
+    return blocks * 4 <= c->num_cus ? 4 : blocks * 2 <= c->num_cus ? 2 : 1;
+}
+
 // Enqueues steps 1-3 on s for M rows of fragment-major codes in the context scratch
 // (d_aq, d_as), leaving the hits at hit_i / hit_s (M x k each) and the list sizes at
 // count (M), all device memory.
@@ -2163,7 +2172,8 @@ int launch_ann_fused(enchip_ctx *c, const Weight &w, int64_t M, int64_t k, hipSt
     int rc;
     const int nk = skinny_shape_nk(w, c->d_aq, w.Kp, true);
     if (!nk && (rc = ensure(c, &c->d_dst, &c->dst_cap, (size_t)(M * kSinkSample) * sizeof(float)))) return rc;
-    const int64_t cand_n = M * (nk ? TOPK_MAXIMA : TOPK_SAMPLE_CHUNKS * k), cap = sink_cap(k);
+    const int64_t parts = maxima_parts(c, M);
+    const int64_t cand_n = M * (nk ? parts * TOPK_MAXIMA : TOPK_SAMPLE_CHUNKS * k), cap = sink_cap(k);
     const size_t words = (size_t)(cand_n + M + M * cap) + (size_t)(M * cap + 1) / 2;
     if ((rc = ensure(c, &c->d_cand, &c->cand_cap, words * sizeof(uint64_t)))) return rc;
     uint64_t *cand = c->d_cand, *thr = cand + cand_n, *keys = thr + M;
@@ -2174,12 +2184,13 @@ int launch_ann_fused(enchip_ctx *c, const Weight &w, int64_t M, int64_t k, hipSt
             const int64_t mr = std::min(most, M - r0);
             const int8_t *aq = c->d_aq + r0 * w.Kp;
             const float *as = c->d_as + r0;
-            uint64_t *mx = cand + r0 * TOPK_MAXIMA;
-            if (mr <= 32) launch_skinny_maxima<1>(w, nk, aq, as, mr, TOPK_MAXIMA, mx, s);
-            else launch_skinny_maxima<2>(w, nk, aq, as, mr, TOPK_MAXIMA, mx, s);
+            uint64_t *mx = cand + r0 * parts * TOPK_MAXIMA;
+            if (mr <= 32) launch_skinny_maxima<1>(w, nk, aq, as, mr, parts, mx, s);
+            else launch_skinny_maxima<2>(w, nk, aq, as, mr, parts, mx, s);
         }
-        hipLaunchKernelGGL(topk_thresh_maxima, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s, (const uint64_t *)cand, M,
-                           (int)k, thr, count);
+        auto *thresh = parts == 4 ? topk_thresh_maxima<4> : parts == 2 ? topk_thresh_maxima<2> : topk_thresh_maxima<1>;
+        hipLaunchKernelGGL(thresh, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s, (const uint64_t *)cand, M, (int)k, thr,
+                           count);
     } else {
         Weight sample = w;
         sample.N = sample.Np = kSinkSample;

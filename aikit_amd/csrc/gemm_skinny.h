@@ -134,65 +134,78 @@ __global__ __launch_bounds__(64 * SK_WAVES, 1) void gemm_w8a8_skinny(
     group(std::false_type{}, n - 1);
 }
 
-// The largest key (topk_key; 0 when all are NaN) of each row's scores in each 32-channel group,
-// maxima[row * groups + group]: the k-th largest of them, the keys of k scores, is a lower bound
-// of the row's k-th largest key, and for k well below the groups nearly the k-th largest of all
-// the scores. Four waves per workgroup take a group each, and RB row blocks (grid.y: 32 RB rows
-// each) whose fragment-major codes lie in LDS; blocks of one x, which read the same weights, run
-// on one XCD. Bound by the maxima's VALU work, so the row blocks are spread over many waves: all
-// 8 blocks of 256 rows in each wave took 32 us. Measured on MI355X for 256 rows, 32768 channels,
-// K = 384, in place of storing the scores (20 us) and selecting from them (18): 17 us.
-constexpr int SM_WAVES = 4;
+// The largest keys (topk_key; 0 when all are NaN) of groups of each row's scores over the sample, the
+// first SM_GROUPS * 32 channels: the k-th largest of them, the keys of k scores, is a lower bound of
+// the row's k-th largest key, and for k well below the groups nearly the k-th largest of all the
+// sample's scores, provided that high scores do not share groups. Rows that lie side by side in an
+// index, the passages of a document say, often score alike, so group j + 32 s (j, s < 32) holds
+// channel c of each 32-channel group j + 32 ((s - c) mod 32): any SM_GROUPS consecutive channels are
+// in different groups, and so are channels a multiple of 32 apart. With groups of 32 adjacent channels
+// and documents of 32 rows (score correlation 0.8, k = 32 over 2^20 rows) the lists came to 4300 of
+// their 4096 places, with these to 1180, as with the k-th largest score itself.
+//
+// Workgroup (j, p, y): the groups of one j, rows 32 RB y ..; its wavefronts and the `parts` (1, 2 or
+// 4) workgroups of one (j, y) share the 32-channel groups j + 32 i, whose scores meet in LDS, a key
+// for every row and s. maxima[(row * parts + p) * SM_GROUPS + 32 j + s]; the parts are left to the
+// reader (topk_thresh_maxima). Workgroups of one j, which read the same weights, run on one XCD.
+// Bound by latency and VALU work, so 32 rows a wavefront at a time and many of them. Measured on
+// MI355X, K = 384, against groups of 32 adjacent channels (whose maxima took five DPP steps a score
+// where a lane's own channel takes one LDS atomic): 16 rows 6.7 -> 5.8 us, 64 rows 10.8 -> 8.7, 256
+// rows 17.2 -> 13.8, 1024 rows 47.7 -> 31.9; K = 512, 256 rows 19.4 -> 17.
+constexpr int SM_WAVES = 8;
+constexpr int SM_GROUPS = TOPK_MAXIMA;
+static_assert(SM_GROUPS == 32 * 32, "32 channel groups of 32 for each of 32 j");
 
 template <int RB, int NK>
-__global__ __launch_bounds__(64 * SM_WAVES) void gemm_w8a8_skinny_maxima(const int8_t *__restrict__ A,
+__global__ __launch_bounds__(64 * SM_WAVES, RB == 1 ? 2 : 4) void gemm_w8a8_skinny_maxima(const int8_t *__restrict__ A,
                                                                             const int8_t *__restrict__ Wf,
                                                                             const float *__restrict__ aS,
                                                                             const float *__restrict__ wS, int M,
-                                                                            uint64_t *__restrict__ maxima) {
+                                                                            int parts, uint64_t *__restrict__ maxima) {
     __shared__ i32x4 s_a[RB * NK * 64];
     __shared__ float s_as[RB * 32];
+    __shared__ unsigned long long s_key[RB * 32 * 32];
     const int tid = threadIdx.x, lane = tid & 63, r0 = blockIdx.y * RB * 32;
-    const int g = blockIdx.x * SM_WAVES + (tid >> 6), groups = gridDim.x * SM_WAVES;
+    const int j = blockIdx.x % 32, p = blockIdx.x / 32, step = parts * SM_WAVES;
+    const int first = p * SM_WAVES + (tid >> 6);
     i32x4 b[NK];
+    float ws = 0.0f;
+    auto load = [&](int i) {
+        const int g = 32 * i + j;
 #pragma unroll
-    for (int kk = 0; kk < NK; ++kk)
-        b[kk] = *reinterpret_cast<const i32x4 *>(Wf + ((int64_t)g * NK + kk) * 1024 + lane * 16);
-    const float ws = wS[g * 32 + (lane & 31)];
+        for (int kk = 0; kk < NK; ++kk)
+            b[kk] = *reinterpret_cast<const i32x4 *>(Wf + ((int64_t)g * NK + kk) * 1024 + lane * 16);
+        ws = wS[g * 32 + (lane & 31)];
+    };
+    load(first);
     const i32x4 *a = reinterpret_cast<const i32x4 *>(A) + (int64_t)blockIdx.y * (RB * NK * 64);
     for (int i = tid; i < RB * NK * 64; i += 64 * SM_WAVES) s_a[i] = a[i];
     for (int r = tid; r < RB * 32; r += 64 * SM_WAVES) s_as[r] = aS[min(r0 + r, M - 1)];
+    for (int i = tid; i < RB * 32 * 32; i += 64 * SM_WAVES) s_key[i] = 0;
     __syncthreads();
-    auto other = [](float x, auto ctrl) {  // another lane of the 16-lane row
-        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
-    };
-    for (int rb = 0; rb < RB; ++rb) {
-        i32x16 acc;
+    for (int i = first; i < 32; i += step) {
+        const float ws_i = ws;
+        const int64_t ch = SM_GROUPS * i + 32 * j + (lane & 31);
+#pragma unroll 1  // one row block's A fragments and sums at a time: with RB = 2, four waves per SIMD
+        for (int rb = 0; rb < RB; ++rb) {
+            i32x16 acc;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] = 0;
+            for (int e = 0; e < 16; ++e) acc[e] = 0;
 #pragma unroll
-        for (int kk = 0; kk < NK; ++kk)
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(s_a[(rb * NK + kk) * 64 + lane], b[kk], acc, 0, 0, 0);
-        uint64_t mine = 0;
+            for (int kk = 0; kk < NK; ++kk)
+                acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(s_a[(rb * NK + kk) * 64 + lane], b[kk], acc, 0, 0, 0);
+            if (rb + 1 == RB && i + step < 32) load(i + step);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const float x = dequant(acc[e], s_as[rb * 32 + acc_row(e, lane)], ws, kNoBias);
-            // the maximum over the lane's half (a NaN only if all are): quad_perm 1,0,3,2 and
-            // 2,3,0,1, row_half_mirror, row_mirror, the other 16-lane row
-            float m = x;
-            m = fmaxf(m, other(m, std::integral_constant<int, 0xB1>{}));
-            m = fmaxf(m, other(m, std::integral_constant<int, 0x4E>{}));
-            m = fmaxf(m, other(m, std::integral_constant<int, 0x141>{}));
-            m = fmaxf(m, other(m, std::integral_constant<int, 0x140>{}));
-            const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-            m = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-            // its first lane; ties (zeros of either sign too) go to the smaller index
-            const uint64_t at = __builtin_amdgcn_ballot_w64(x == m);
-            const uint32_t half = lane < 32 ? (uint32_t)at : (uint32_t)(at >> 32);
-            if ((lane & 31) == e && half != 0u) mine = topk_key(m, g * 32 + __builtin_ctz(half));
+            for (int e = 0; e < 16; ++e) {
+                const int row = rb * 32 + acc_row(e, lane);
+                atomicMax(&s_key[row * 32 + ((lane + i) & 31)], topk_key(dequant(acc[e], s_as[row], ws_i, kNoBias), ch));
+            }
         }
-        const int row = r0 + rb * 32 + acc_row(lane & 15, lane);
-        if ((lane & 31) < 16 && row < M) maxima[(int64_t)row * groups + g] = mine;
+    }
+    __syncthreads();
+    for (int i = tid; i < RB * 32 * 32; i += 64 * SM_WAVES) {
+        const int row = r0 + i / 32;
+        if (row < M) maxima[((int64_t)row * parts + p) * SM_GROUPS + 32 * j + i % 32] = s_key[i];
     }
 }
 

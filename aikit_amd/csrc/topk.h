@@ -595,19 +595,29 @@ __global__ __launch_bounds__(256) void topk_thresh_sorted(const uint64_t *__rest
 }
 
 // The row thresholds from the maxima of TOPK_MAXIMA groups of a row's scores (keys, 0 for a group
-// of NaN): the k-th largest of them, or 0 when fewer than k are nonzero. One wavefront per row
-// searches it bit by bit, counting by ballot, and stops at a value that exactly k keys reach.
+// of NaN; the largest of PARTS for each group, maxima[(row * PARTS + part) * TOPK_MAXIMA + group]):
+// the k-th largest of them, or 0 when fewer than k are nonzero. One wavefront per row searches it
+// bit by bit, counting by ballot, and stops at a value that exactly k keys reach.
 constexpr int TOPK_MAXIMA = TOPK_SAMPLE_CHUNKS * TOPK_WCHUNK / 32;
 
+template <int PARTS>
 __global__ __launch_bounds__(256) void topk_thresh_maxima(const uint64_t *__restrict__ maxima, int64_t rows, int k,
                                                           uint64_t *__restrict__ thr, unsigned *__restrict__ zero) {
     constexpr int PER_LANE = TOPK_MAXIMA / 64;
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    uint64_t v[PER_LANE];
+    uint64_t x[PARTS][PER_LANE], v[PER_LANE];
 #pragma unroll
-    for (int i = 0; i < PER_LANE; ++i) v[i] = maxima[row * TOPK_MAXIMA + lane + 64 * i];
+    for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) x[p][i] = maxima[(row * PARTS + p) * TOPK_MAXIMA + lane + 64 * i];
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+        v[i] = x[0][i];
+#pragma unroll
+        for (int p = 1; p < PARTS; ++p) v[i] = max(v[i], x[p][i]);
+    }
     uint64_t t = 0;  // at least k keys are >= t, once it is not 0
     int n = 0;
     for (int bit = 31; bit >= 0 && n != k; --bit) {  // the scores' bits

@@ -78,3 +78,38 @@ def test_bounds_of_few_live_groups(ctx, k, live):
         idx, sc = oracle.top_hits(scores[r], k)
         assert hi[r].tolist() == idx.tolist(), f"row {r}: indices differ"
         assert np.array_equal(hs[r].view(np.uint32), sc.view(np.uint32)), f"row {r}: scores differ"
+
+
+@pytest.mark.parametrize("M,N,K,k,doc", [(8, 1 << 20, 128, 32, 32), (40, 1 << 20, 128, 32, 16), (130, 1 << 19, 128, 64, 32)])
+def test_rows_stored_by_document_stay_on_the_fused_route(ctx, M, N, K, k, doc):
+    # `doc` consecutive rows score alike (correlation 0.9), as the passages of a document stored in
+    # order do: the bounds are as tight as over any order, so the lists hold and the fused route
+    # answers. Taken over 32 adjacent columns the group maxima would let too many through.
+    g = workloads.rng(8100 + M + doc)
+    x = np.repeat(g.standard_normal((N // doc, K), dtype=np.float32), doc, axis=0) * np.float32(0.9**0.5)
+    x += g.standard_normal((N, K), dtype=np.float32) * np.float32(0.1**0.5)
+    codes = np.clip(np.rint(x * 30), -127, 127).astype(np.int8)
+    del x
+    scales = np.full(N, 1e-3, np.float32)
+    q = g.standard_normal((M, K)).astype(np.float32)
+    print(f"[case] ann by document M={M} N={N} K={K} k={k} doc={doc}", flush=True)
+    w = ctx.register_weight(codes, scales)
+    try:
+        f0, b0 = ctx.ann_topk_stats()
+        hi, hs = ctx.ann_topk(w, q, k)
+        f1, b1 = ctx.ann_topk_stats()
+    finally:
+        ctx.release_weight(w)
+    scores = oracle.w8a8_linear(q, codes, scales, None, 0, M, K, N)
+    sample, cap = scores[:, :32768], 4096 if k <= 32 else 8192
+
+    def longest(groups):
+        kth = -np.partition(-groups, k - 1, axis=1)[:, k - 1]
+        return int((scores >= kth[:, None]).sum(axis=1).max())
+
+    assert longest(sample) <= cap < longest(sample.reshape(M, 1024, 32).max(axis=2)), "the case"
+    assert (f1 - f0, b1 - b0) == (1, 0), "route"
+    for r in range(M):
+        idx, sc = oracle.top_hits(scores[r], k)
+        assert hi[r].tolist() == idx.tolist(), f"row {r}: indices differ"
+        assert np.array_equal(hs[r].view(np.uint32), sc.view(np.uint32)), f"row {r}: scores differ"
