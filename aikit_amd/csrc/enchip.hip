@@ -129,11 +129,11 @@ struct enchip_ctx {
     // capped at scratch_limit bytes (enchip_set_scratch_limit; 0 = no cap).
     size_t scratch_limit = 0;
     // The last stream that enqueued work on the shared scratch (d_aq, d_as, d_cand) and
-    // an event recorded after that work: a user on another stream waits for it first. After
-    // work on the context's own stream the event is recorded only when such a user comes.
+    // an event recorded after that work: a user on another stream waits for it first. Until the
+    // first such user comes, work on the context's own stream records none.
     hipEvent_t scratch_ev = nullptr;
     hipStream_t scratch_stream = nullptr;
-    bool scratch_pending = false, scratch_recorded = false;
+    bool scratch_pending = false, scratch_recorded = false, scratch_shared = false;
     int8_t *d_aq = nullptr;
     size_t aq_cap = 0;
     float *d_as = nullptr;
@@ -347,7 +347,8 @@ int download(enchip_ctx *c, void *dst, const void *src, size_t bytes, hipStream_
 int scratch_wait(enchip_ctx *c, hipStream_t s) {
     if (!c->scratch_pending || c->scratch_stream == s || capturing(s)) return ENCHIP_OK;
     hipError_t e;
-    if (!c->scratch_recorded) {  // the last user was the context's stream
+    c->scratch_shared = true;
+    if (!c->scratch_recorded) {  // the last user was the context's stream, alone so far
         if ((e = hipEventRecord(c->scratch_ev, c->stream)) != hipSuccess)
             return fail(c, ENCHIP_ERR_HIP, "hipEventRecord(scratch): %s", hipGetErrorString(e));
         c->scratch_recorded = true;
@@ -359,16 +360,19 @@ int scratch_wait(enchip_ctx *c, hipStream_t s) {
 
 // Marks the scratch as in use by the work just enqueued on stream s. An event costs the
 // stream about 5 us on MI355X (a 512-row linear's two launches 12.7 us per call with it, 9.5
-// without), so work on the context's own stream, which lives as long as the scratch and is
-// captured by nobody, leaves it to the next user on another stream (scratch_wait). A caller's
-// stream may be gone by then: its event is recorded here.
+// without), so while no other stream has waited for the scratch, work on the context's own
+// stream, which lives as long as the scratch and is captured by nobody, leaves it to the first
+// that does (scratch_wait; that one waits for all the work enqueued there so far). From then on,
+// and after work on a caller's stream, which may be gone by the next use, it is recorded here:
+// another stream waits for the scratch's last use and for nothing after it.
 int scratch_record(enchip_ctx *c, hipStream_t s) {
-    if (s != c->stream) {
-        if (capturing(s)) return ENCHIP_OK;
+    const bool record = s != c->stream || c->scratch_shared;
+    if (record) {
+        if (s != c->stream && capturing(s)) return ENCHIP_OK;
         hipError_t e = hipEventRecord(c->scratch_ev, s);
         if (e != hipSuccess) return fail(c, ENCHIP_ERR_HIP, "hipEventRecord(scratch): %s", hipGetErrorString(e));
     }
-    c->scratch_recorded = s != c->stream;
+    c->scratch_recorded = record;
     c->scratch_stream = s;
     c->scratch_pending = true;
     return ENCHIP_OK;
