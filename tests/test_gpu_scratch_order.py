@@ -1,6 +1,7 @@
 """GPU test of the shared scratch's ordering between the context's own stream and others: calls
 that quantize into it, enqueued back to back on alternating streams, give the results of the
 same calls one at a time."""
+import ctypes
 import time
 
 import pytest
@@ -28,11 +29,81 @@ def test_alternating_streams_share_the_scratch():
         for rep in range(5):
             for x, y, o in zip(a, out, order):
                 c.linear_dev(w, x.data_ptr(), M, 0, enchip.ACT_NONE, y.data_ptr(), 0 if o == 0 else others[o - 1].cuda_stream)
-        del others[1]  # a caller's stream may go before the scratch is used again
         c.linear_dev(w, a[0].data_ptr(), M, 0, enchip.ACT_NONE, out[0].data_ptr())
         torch.cuda.synchronize()
         for y, z in zip(out, want):
             assert torch.equal(y.view(torch.int32), z.view(torch.int32))
+
+
+def hip():
+    """The HIP runtime this process has loaded."""
+    with open("/proc/self/maps") as f:
+        return ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_a_stream_that_is_gone_was_the_last_user(first):
+    # A caller's stream uses the scratch last and is destroyed before the context's stream uses it
+    # again: before any use on the context's stream, or after one.
+    import torch
+
+    g = workloads.rng(33)
+    M, K, N = 3000, 1024, 1024
+    with enchip.Context(0) as c:
+        w = c.register_weight(*workloads.int8_weights(g, N, K))
+        a = [torch.from_numpy(workloads.activations(g, M, K)).cuda() for _ in range(3)]
+        out, want = ([torch.empty((M, N), device="cuda") for _ in a] for _ in range(2))
+        torch.cuda.synchronize()
+        with enchip.Context(0) as alone:
+            w1 = alone.register_weight(*workloads.int8_weights(workloads.rng(33), N, K))
+            for x, y in zip(a, want):
+                alone.linear_dev(w1, x.data_ptr(), M, 0, enchip.ACT_NONE, y.data_ptr())
+                torch.cuda.synchronize()
+        lib, s = hip(), ctypes.c_void_p()
+        for rep in range(5):
+            if not first:
+                c.linear_dev(w, a[0].data_ptr(), M, 0, enchip.ACT_NONE, out[0].data_ptr())
+            assert lib.hipStreamCreate(ctypes.byref(s)) == 0
+            print(f"[case] scratch and a destroyed stream, first={first} rep={rep}", flush=True)
+            c.linear_dev(w, a[1].data_ptr(), M, 0, enchip.ACT_NONE, out[1].data_ptr(), s.value)
+            assert lib.hipStreamDestroy(s) == 0
+            c.linear_dev(w, a[2].data_ptr(), M, 0, enchip.ACT_NONE, out[2].data_ptr())
+            torch.cuda.synchronize()
+            for i in range(int(first), 3):
+                assert torch.equal(out[i].view(torch.int32), want[i].view(torch.int32))
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_the_scratch_grows_while_in_use(shared):
+    # Work on the context's stream (with no event, or with one where another stream has used the
+    # scratch) reads the scratch when a call with more rows replaces it.
+    import torch
+
+    g = workloads.rng(34)
+    K, N = 1024, 1024
+    Ms = [2000, 6000, 14000]
+    a = [torch.from_numpy(workloads.activations(g, M, K)).cuda() for M in Ms]
+    wq, ws = workloads.int8_weights(g, N, K)
+    got = []
+    for wait in (True, False):
+        with enchip.Context(0) as c:
+            w = c.register_weight(wq, ws)
+            outs = [torch.empty((M, N), device="cuda") for M in Ms]
+            s = torch.cuda.Stream()
+            torch.cuda.synchronize()
+            print(f"[case] scratch growth shared={shared} wait={wait}", flush=True)
+            if shared:
+                for stream in (0, s.cuda_stream):
+                    c.linear_dev(w, a[0].data_ptr(), 100, 0, enchip.ACT_NONE, outs[0].data_ptr(), stream)
+                torch.cuda.synchronize()
+            for M, x, y in zip(Ms, a, outs):
+                c.linear_dev(w, x.data_ptr(), M, 0, enchip.ACT_NONE, y.data_ptr())
+                if wait:
+                    torch.cuda.synchronize()
+            torch.cuda.synchronize()
+            got.append(outs)
+    for x, y in zip(*got):
+        assert torch.equal(x.view(torch.int32), y.view(torch.int32))
 
 
 def test_another_stream_waits_for_the_scratch_alone():
