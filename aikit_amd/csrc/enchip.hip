@@ -255,16 +255,16 @@ constexpr size_t kDownSlice = (size_t)512 << 10, kDownHalf = 4 * kDownSlice;
 constexpr size_t kStageBytes = 2 * kDownHalf, kStageWords = 2 * (kDownHalf / kDownSlice) * enchip::COPY_OUT_BLOCKS;
 static_assert(2 * kStageChunk <= kStageBytes, "upload's slots lie in the staging");
 
+// Where pinned memory cannot be had, h_stage stays null and the copies are pageable.
 int ensure_stage(enchip_ctx *c) {
     if (c->h_stage) return ENCHIP_OK;
     for (hipEvent_t &e : c->stage_ev)
         if (!e) HIP_TRY(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     void *p = nullptr;
     const size_t bytes = kStageBytes + kStageWords * sizeof(uint32_t);
-    hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocCoherent);  // copy_out's stores are polled
-    if (e != hipSuccess) {
+    if (hipHostMalloc(&p, bytes, hipHostMallocCoherent) != hipSuccess) {  // copy_out's stores are polled
         (void)hipGetLastError();
-        return fail(c, ENCHIP_ERR_OOM, "hipHostMalloc(%zu): %s", bytes, hipGetErrorString(e));
+        return ENCHIP_OK;
     }
     c->h_stage = static_cast<char *>(p);
     std::memset(c->h_stage + kStageBytes, 0, kStageWords * sizeof(uint32_t));
@@ -274,12 +274,12 @@ int ensure_stage(enchip_ctx *c) {
 // Enqueues the copy of `bytes` from host memory src to device memory dst on s. src may be
 // reused once this returns (every byte is in a pinned slot or already on its way).
 int upload(enchip_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < kStageMinUp) {
+    int rc;
+    if (bytes >= kStageMinUp && (rc = ensure_stage(c))) return rc;
+    if (bytes < kStageMinUp || !c->h_stage) {
         if (bytes) HIP_TRY(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
         return ENCHIP_OK;
     }
-    int rc;
-    if ((rc = ensure_stage(c))) return rc;
     for (size_t off = 0, i = 0; off < bytes; off += kStageChunk, ++i) {
         const size_t n = std::min(kStageChunk, bytes - off);
         char *slot = c->h_stage + (i & 1) * kStageChunk;
@@ -292,15 +292,15 @@ int upload(enchip_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t 
 }
 
 // Copies `bytes` from device memory src (16-byte aligned) to host memory dst after the work
-// already enqueued on s. A small copy is only enqueued (the caller synchronizes s before it reads
+// already enqueued on s. A pageable copy is only enqueued (the caller synchronizes s before it reads
 // dst); a staged one has completed when this returns.
 int download(enchip_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < kStageMinDown) {
+    int rc;
+    if (bytes >= kStageMinDown && (rc = ensure_stage(c))) return rc;
+    if (bytes < kStageMinDown || !c->h_stage) {
         if (bytes) HIP_TRY(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         return ENCHIP_OK;
     }
-    int rc;
-    if ((rc = ensure_stage(c))) return rc;
     for (hipEvent_t e : c->stage_ev) HIP_TRY(c, hipEventSynchronize(e));  // earlier uploads' DMAs
     // launch l moves bytes [l kDownHalf, ..) into half l % 2, two launches ahead of the CPU
     const size_t launches = (bytes + kDownHalf - 1) / kDownHalf;
@@ -2260,8 +2260,8 @@ int fetch_hits(enchip_ctx *c, hipStream_t s, int64_t M, int64_t k, int32_t *hit_
     int rc;
     std::vector<char> big;
     const char *host;
-    if (bytes <= kStageChunk) {
-        if ((rc = ensure_stage(c))) return rc;
+    if (bytes <= kStageChunk && (rc = ensure_stage(c))) return rc;
+    if (bytes <= kStageChunk && c->h_stage) {
         for (hipEvent_t e : c->stage_ev) HIP_TRY(c, hipEventSynchronize(e));  // no DMA still reads a slot
         HIP_TRY(c, hipMemcpyAsync(c->h_stage, c->d_hits, bytes, hipMemcpyDeviceToHost, s));
         HIP_TRY(c, hipStreamSynchronize(s));

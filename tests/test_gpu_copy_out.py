@@ -1,5 +1,9 @@
 """GPU tests of the staged copy of results to host memory at the edges of its slices (512 KiB),
 halves (2 MiB) and launches: every byte, from several threads and contexts."""
+import inspect
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -57,3 +61,44 @@ def test_threads_and_contexts(ctx):
         t.join()
     other.close()
     assert not errors, errors
+
+
+def host_calls(ctx):
+    # results of 600 KiB and of 3 MiB, inputs of 6 MiB, top-k hits
+    g = workloads.rng(55)
+    out = []
+    for M, K, N in ((200, 64, 768), (1536, 1024, 512)):
+        w = ctx.register_weight(*workloads.int8_weights(g, N, K))
+        out.append(ctx.linear(w, workloads.activations(g, M, K)))
+    out += list(ctx.quant_rows(workloads.activations(g, 1100, 512)))
+    out.append(ctx.matmul_bt_f32(workloads.activations(g, 300, 96), workloads.activations(g, 700, 96)))
+    out += list(ctx.ann_topk(w, workloads.activations(g, 5, 1024), 7))
+    return out
+
+
+SHIM = "int hipHostMalloc(void **p, unsigned long n, unsigned f) { if (p) *p = 0; ++calls; return 2; }"
+
+
+def test_without_pinned_memory_the_copies_are_pageable(ctx, tmp_path):
+    # A process whose pinned allocations fail (a hipHostMalloc that answers out of memory stands
+    # before the runtime's) gets the results of one that has them.
+    (tmp_path / "shim.c").write_text("int calls;\n" + SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "shim.so"), str(tmp_path / "shim.c")], check=True)
+    child = f"""
+import ctypes
+shim = ctypes.CDLL({str(tmp_path / 'shim.so')!r}, mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+from aikit_amd import enchip, workloads
+{inspect.getsource(host_calls)}
+with enchip.Context(0) as c:
+    out = host_calls(c)
+assert ctypes.c_int.in_dll(shim, "calls").value > 0, "the library's allocations did not fail"
+np.savez({str(tmp_path / 'out.npz')!r}, *out)
+"""
+    print("[case] host copies without pinned memory", flush=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", child], cwd=root, timeout=100, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    with np.load(tmp_path / "out.npz") as got:
+        for i, want in enumerate(host_calls(ctx)):
+            assert np.array_equal(got[f"arr_{i}"].view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), i
