@@ -25,7 +25,7 @@
 // 3.9e-7 with, as on the f32 MFMA throughout. The looking costs up to 3%: 4096 x 768, K = 768 40.0 ->
 // 41.3 us, 512 x 3072 25.4 -> 26.0, 4096 x 3072, K = 3072 391 -> 395, K-split shapes none.
 // An operand the split cannot hold (an infinity, or a value that rounds to one in bf16) or a
-// sum that overflows leaves a non-finite output; those are computed again by f32_block on the f32
+// sum that overflows leaves a non-finite output; those are computed again by f32_blocks on the f32
 // MFMA, so infinities and overflow give what f32 arithmetic gives. The other outputs of the block
 // keep their split sums.
 //
@@ -96,7 +96,7 @@ __device__ __forceinline__ void mfma_parts(const bf16x8 (&pa)[TM][3], const bf16
 // sum of K products with every operand at most kBig then lost at most 2 K 2^-134 kBig = K 2^-109,
 // under 2^-25 of any output from lost_below(K) up. So the main loop only looks for operands above
 // kBig, and the end for outputs below that (zeros, as a rule): blocks with either have their
-// operands searched for small ones, and f32_block computes the outputs that can have lost by it.
+// operands searched for small ones, and f32_blocks computes the outputs that can have lost by it.
 // (Looking for the small ones in the main loop cost up to 12%.)
 constexpr uint32_t kBelow = ((127u - 110u) << 24) - 1u;
 constexpr float kBig = 0x1p24f;
@@ -119,63 +119,127 @@ __device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN], float
     return s != 0.0f;  // 0, or NaN
 }
 
-// Whether a nonzero value under 2^-110 is among the `rows` rows at p (pitch ld, n values each), by
-// one wavefront.
-__device__ __forceinline__ bool holds_small(const float *p, int64_t ld, int rows, int n) {
-    uint32_t low = ~0u;
-    for (int i = 0; i < rows; ++i)
-        for (int k = threadIdx.x & 63; k < n; k += 64) low = min(low, below_split(p[i * ld + k]));
-    return __builtin_amdgcn_ballot_w64(low < kBelow) != 0;
-}
-
-template <bool BKN>
-__device__ __forceinline__ bool operands_small(const float *A, int64_t lda, const float *B, int64_t ldb, int M, int N, int K,
-                                            int m0, int n0, int rows, int cols) {
-    const int m = min(rows, M - m0), n = min(cols, N - n0);
-    if (m <= 0 || n <= 0) return false;
-    return holds_small(A + (int64_t)m0 * lda, lda, m, K) ||
-           (BKN ? holds_small(B + n0, ldb, K, n) : holds_small(B + (int64_t)n0 * ldb, ldb, n, K));
-}
-
-// The 32 x 32 outputs at (m0, n0), stored from split sums, computed by one wavefront on the f32
-// MFMA with operands loaded value by value, and stored where the split sum is not finite or can have
-// lost by a small operand: whatever the tile, each output by its own row, column and split sum.
-template <bool BKN>
-__device__ __forceinline__ void f32_block(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc,
-                                       int M, int N, int K, int m0, int n0) {
-    const int lane = threadIdx.x & 63, r = lane & 31, kh = 8 * (lane >> 5);
-    if (m0 >= M || n0 >= N) return;
-    const float *pa = A + (int64_t)min(m0 + r, M - 1) * lda;
-    const int n = min(n0 + r, N - 1);
-    f32x16 acc;
+// For up to 32 rows of n values (row i at p + i * pitch, value k at k * step; those in mask), by one
+// wavefront: which hold a nonzero value, one under 2^-110, one above kBig. Four rows at a time, for
+// the loads in flight.
+struct RowMarks {
+    uint32_t live, small, big;
+};
+__device__ __forceinline__ RowMarks row_marks(const float *p, int64_t pitch, int64_t step, int n, uint32_t mask) {
+    constexpr int R = 4, U = 4;
+    const int lane = threadIdx.x & 63;
+    RowMarks marks{0, 0, 0};
+    while (mask != 0) {  // uniform
+        int row[R];
+        float most[R];
+        uint32_t low[R];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-    float big_a = 0.0f, big_b = 0.0f;  // of row m0 + r, of column n0 + r
-    uint32_t low_a = ~0u, low_b = ~0u;
-    for (int k0 = 0; k0 < K; k0 += 16) {
+        for (int q = 0; q < R; ++q) {
+            row[q] = __builtin_ctz(mask);
+            if ((mask & (mask - 1)) != 0 || q == R - 1) mask &= mask - 1;  // else the last row again
+            most[q] = 0.0f, low[q] = ~0u;
+        }
+        for (int k0 = 0; k0 < n; k0 += 64 * U) {
+            float x[R][U];
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const int k = k0 + kh + s, kc = min(k, K - 1);
-            const float av = pa[kc], bv = BKN ? B[(int64_t)kc * ldb + n] : B[(int64_t)n * ldb + kc];
-            const float a = k < K ? av : 0.0f, b = k < K ? bv : 0.0f;
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-            big_a = fmaxf(big_a, fabsf(a)), big_b = fmaxf(big_b, fabsf(b));
-            low_a = min(low_a, below_split(a)), low_b = min(low_b, below_split(b));
+            for (int q = 0; q < R; ++q)
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[q][u] = p[row[q] * pitch + min(k0 + 64 * u + lane, n - 1) * step];
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    most[q] = fmaxf(fabsf(x[q][u]), most[q]);
+                    low[q] = min(below_split(x[q][u]), low[q]);
+                }
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const uint32_t bit = 1u << row[q];
+            if (__builtin_amdgcn_ballot_w64(most[q] > 0.0f) != 0) marks.live |= bit;
+            if (__builtin_amdgcn_ballot_w64(low[q] < kBelow) != 0) marks.small |= bit;
+            if (__builtin_amdgcn_ballot_w64(most[q] > kBig) != 0) marks.big |= bit;
         }
     }
-    big_a = fmaxf(big_a, __shfl_xor(big_a, 32)), big_b = fmaxf(big_b, __shfl_xor(big_b, 32));
-    low_a = min(low_a, (uint32_t)__shfl_xor((int)low_a, 32)), low_b = min(low_b, (uint32_t)__shfl_xor((int)low_b, 32));
-    const float small_out = lost_below(K);
+    return marks;
+}
+
+// Of the lane's 16 outputs of a 32 x 32 block, a bit each: those not finite, those under lost_below.
+struct OutMarks {
+    uint32_t bad, low;
+};
+__device__ __forceinline__ OutMarks out_marks(const f32x16 &v, int K) {
+    OutMarks o{0, 0};
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-        const int at = acc_row(e, lane), row = m0 + at;
-        const float ba = __shfl(big_a, at);
-        const uint32_t la = (uint32_t)__shfl((int)low_a, at);
-        if (row >= M || n0 + r >= N) continue;
-        float *c = C + (int64_t)row * ldc + n0 + r;
-        const float old = *c;
-        const bool lost = min(la, low_b) < kBelow && (fabsf(old) < small_out || fmaxf(ba, big_b) > kBig);
-        if (lost || !(fabsf(old) < INFINITY)) *c = acc[e];
+        o.bad |= (uint32_t)!(fabsf(v[e]) < INFINITY) << e;
+        o.low |= (uint32_t)(fabsf(v[e]) < lost_below(K)) << e;
+    }
+    return o;
+}
+
+// The TN 32 x 32 outputs at (m0, n0), (m0, n0 + 32), ..., stored from split sums, by one wavefront:
+// those not finite, and those that can have lost by a small operand of their row or column, are
+// computed again on the f32 MFMA with operands loaded value by value. Which ones depends on each
+// output's own row, column and split sum, whatever the tile. any_big: the block has an operand above
+// kBig. Rows of zeros, whose outputs are under lost_below, need no search of the columns.
+template <int TN, bool BKN>
+__device__ __forceinline__ void f32_blocks(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc,
+                                        int M, int N, int K, int m0, int n0, bool any_big, const OutMarks (&marks)[TN]) {
+    const int lane = threadIdx.x & 63, r = lane & 31, kh = 8 * (lane >> 5);
+    if (m0 >= M) return;
+    uint32_t in_rows = 0, doubt[TN], rows = 0;  // doubt: the lane's outputs that can have lost; rows: with any
+#pragma unroll
+    for (int e = 0; e < 16; ++e) in_rows |= (uint32_t)(m0 + acc_row(e, lane) < M) << e;
+    uint32_t any = 0;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        doubt[t] = n0 + 32 * t + r < N ? (any_big ? ~0u : marks[t].low) & in_rows : 0;
+        any |= doubt[t];
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const uint64_t b = __builtin_amdgcn_ballot_w64((any >> e) & 1);
+        rows |= (uint32_t)((uint32_t)b != 0) << acc_row(e, 0) | (uint32_t)((b >> 32) != 0) << acc_row(e, 32);
+    }
+    const RowMarks ra = row_marks(A + (int64_t)m0 * lda, lda, 1, K, rows);
+#pragma unroll 1
+    for (int t = 0; t < TN; ++t, n0 += 32) {
+        uint32_t dt = doubt[0], low = marks[0].low, redo = marks[0].bad;
+#pragma unroll
+        for (int u = 1; u < TN; ++u)
+            if (t == u) dt = doubt[u], low = marks[u].low, redo = marks[u].bad;
+        redo &= n0 + r < N ? in_rows : 0;
+        bool col = false;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) col |= ((dt >> e) & (ra.live >> acc_row(e, lane)) & 1) != 0;
+        if (__builtin_amdgcn_ballot_w64(col || redo != 0) == 0) continue;
+        const uint64_t cb = __builtin_amdgcn_ballot_w64(col);
+        const RowMarks rb = BKN ? row_marks(B + n0, 1, ldb, K, (uint32_t)cb | (uint32_t)(cb >> 32))
+                                : row_marks(B + (int64_t)n0 * ldb, ldb, 1, K, (uint32_t)cb | (uint32_t)(cb >> 32));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int at = acc_row(e, lane);
+            const uint32_t small = ra.small >> at | rb.small >> r, big = ra.big >> at | rb.big >> r;
+            redo |= (dt >> e & small & (low >> e | big) & 1) << e;
+        }
+        if (__builtin_amdgcn_ballot_w64(redo != 0) == 0) continue;
+        const float *pa = A + (int64_t)min(m0 + r, M - 1) * lda;
+        const int n = min(n0 + r, N - 1);
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+        for (int k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const int k = k0 + kh + s, kc = min(k, K - 1);
+                const float a = pa[kc], b = BKN ? B[(int64_t)kc * ldb + n] : B[(int64_t)n * ldb + kc];
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < K ? a : 0.0f, k < K ? b : 0.0f, acc, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if ((redo >> e) & 1) C[(int64_t)(m0 + acc_row(e, lane)) * ldc + n0 + r] = acc[e];
     }
 }
 
@@ -338,11 +402,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
         for (int s = 0; s < KC / 16; ++s) mfma_parts<TM, TN>(pa[s], pb[s], acc);
         lds_barrier();
     }
+    // The last loads, of a chunk already used, end here: left in flight, their registers' next use
+    // waits in each store's branch, for the stores before it too (16 x 64 problems 3.6 -> 4.1 us).
+#pragma unroll
+    for (int i = 0; i < AV; ++i) asm volatile("" ::"v"(ra[i]));
+#pragma unroll
+    for (int i = 0; i < BV; ++i) asm volatile("" ::"v"(rb[i]));
     if (big > kBig) any_big = 1;
     lds_barrier();
     float least = INFINITY;
     const bool nonfinite = __builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc, least)) != 0;
-    const bool doubt = any_big != 0 || __builtin_amdgcn_ballot_w64(least < lost_below(K)) != 0;
+    const bool low = __builtin_amdgcn_ballot_w64(least < lost_below(K)) != 0;
     const int m0 = bm0 + 32 * TM * wm, n0 = bn0 + 32 * TN * wn;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -356,10 +426,24 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
                 if (row < M) C[(int64_t)row * ldc + col] = acc[i][t][e];
             }
         }
-    if (__builtin_expect(nonfinite || doubt, 0)) {
-        if (nonfinite || operands_small<BKN>(A, lda, B, ldb, M, N, K, m0, n0, 32 * TM, 32 * TN))
-            for (int u = 0; u < TM * TN; ++u)
-                f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * (u / TN), n0 + 32 * (u % TN));
+    if (__builtin_expect(nonfinite || low || any_big != 0, 0)) {
+        OutMarks marks[TM][TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) marks[i][t] = out_marks(acc[i][t], K);
+#pragma unroll 1
+        for (int i = 0; i < TM; ++i) {
+            OutMarks mi[TN];
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                mi[t] = marks[0][t];
+#pragma unroll
+                for (int u = 1; u < TM; ++u)
+                    if (i == u) mi[t] = marks[u][t];
+            }
+            f32_blocks<TN, BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + 32 * i, n0, any_big != 0, mi);
+        }
     }
 }
 
@@ -473,7 +557,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
             for (int e = 0; e < 16; ++e) red[wave][(32 * i + acc_row(e, lane)) * P + 32 * t + r] = acc[i][t][e];
     __syncthreads();
     constexpr int RL = BN / 4, RP = NT / RL, NG = BM * RL / NT;  // 16-byte groups per row; rows per pass; passes
-    static_assert(BM * RL % NT == 0, "whole passes");
+    static_assert(BM * RL % NT == 0 && WK == 4, "whole passes");
     const int c4 = 4 * (tid % RL), r0 = tid / RL, col = n0 + c4;
     const bool vst = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C & 15) == 0;
     float zeros = 0.0f, least = INFINITY;  // of the sums: NaN where one is not finite; the smallest
@@ -502,13 +586,18 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ksplit(const float *__restric
                 if (col + u < N) o[u] = x[u];
         }
     }
-    const bool nonfinite = zeros != 0.0f;
-    if (__builtin_expect(__syncthreads_or(nonfinite || big > kBig || least < lost_below(K)), 0)) {
-        const bool redo = __syncthreads_or(nonfinite);
+    if (__builtin_expect(__syncthreads_or(zeros != 0.0f || big > kBig || least < lost_below(K)), 0)) {
+        const bool any_big = __syncthreads_or(big > kBig);
         for (int u = wave; u < TM * TN; u += WK) {
-            const int mu = m0 + 32 * (u / TN), nu = n0 + 32 * (u % TN);
-            if (redo || operands_small<BKN>(A, lda, B, ldb, M, N, K, mu, nu, 32, 32))
-                f32_block<BKN>(A, lda, B, ldb, C, ldc, M, N, K, mu, nu);
+            const int mu = 32 * (u / TN), nu = 32 * (u % TN);
+            f32x16 v;  // the sums again, each lane its f32 MFMA outputs
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int at = (mu + acc_row(e, lane)) * P + nu + r;
+                v[e] = ((red[0][at] + red[1][at]) + red[2][at]) + red[3][at];
+            }
+            const OutMarks marks[1] = {out_marks(v, K)};
+            f32_blocks<1, BKN>(A, lda, B, ldb, C, ldc, M, N, K, m0 + mu, n0 + nu, any_big, marks);
         }
     }
 }
