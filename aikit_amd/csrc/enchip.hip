@@ -1561,7 +1561,9 @@ int launch_matmul_f32(enchip_ctx *c, const float *A, int64_t lda, const float *B
     // 512 x 768, K = 768 (96 tiles) 12.0 us against 18.1; 512 x 3072 (384) 32.2 against 22.9.
     // Narrow outputs (scores . V) come in batches, where the tiles are faster: 512 x 64, K =
     // 512 over 384 heads 142 against 134. Tile sizes, by the launch's number of tiles: the
-    // largest that still give every CU work (the kernels' comments have the figures).
+    // largest that still give every CU work (the kernels' comments have the figures), and no taller
+    // than the problem: 16 x 100000, K = 768 96 us in 64 x 64 tiles against 145 in 128 x 64, 64 x 64
+    // x 64 over 1536 heads 18.3 against 24.2.
     const int64_t cus = c->num_cus, nb = b1.count * b2.count;
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const bool ksplit = K >= 256 && N > 128 && tiles(64, 64) <= cus / 2;
@@ -1574,7 +1576,7 @@ int launch_matmul_f32(enchip_ctx *c, const float *A, int64_t lda, const float *B
     } else if (N > 64 && tiles(64, 128) * nb > cus / 2 && tiles(64, 128) * nb <= cus) {
         bm = 64, bn = 128;
     } else {
-        bm = tiles(64, 64) * nb > 2 * cus ? 128 : 64, bn = 64;
+        bm = M > 64 && tiles(64, 64) * nb > 2 * cus ? 128 : 64, bn = 64;
     }
     // Columns per launch: with M * N <= 2^36 every launch's threads then stay below 2^32 (only
     // M <= 128 has more columns).
