@@ -1710,7 +1710,9 @@ int launch_matmul_q8w(enchip_ctx *c, const Weight &w, const float *A, int64_t ld
     const bool vec = w.K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0;
     // The K-split small form while there is at most one of its 32 x 32 tiles per CU: M = 64, K
     // = 768, N = 3072 (192 tiles) takes 9.3 us against 11.1 in 32 x 128 tiles, M = 128, N =
-    // 2304 (288) 12.0 against 11.2. 128 x 256 tiles when they fill the CUs: about one each, or
+    // 2304 (288) 12.0 against 11.2; up to two where A's rows are not 16-byte aligned (K = 1001: M =
+    // 300, N = 1000, 320 tiles, 12.8 against 14.4, M = 512 13.4 against 14.9, M = 700 19.5 against
+    // 15.2). 128 x 256 tiles when they fill the CUs: about one each, or
     // from one and a half (in between, the second round is mostly empty): M = 2048, K = 1024,
     // N = 4096 (256 tiles) 54 us against 65 in 32 x 128, M = 4096, K = 768, N = 2304 (288) 63
     // against 56, N = 3072 (384) 66 against 72. Otherwise 32 x 128, K in chunks of 128 while
@@ -1718,7 +1720,7 @@ int launch_matmul_q8w(enchip_ctx *c, const Weight &w, const float *A, int64_t ld
     const int64_t cus = c->num_cus;
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((w.N + bn - 1) / bn); };
     const int64_t big = tiles(128, 256);
-    const int form = tiles(32, 32) <= cus                                            ? 0
+    const int form = tiles(32, 32) <= (vec ? 1 : 2) * cus                            ? 0
                      : 4 * big >= 3 * cus && (big <= cus || 2 * big >= 3 * cus) ? 3
                      : tiles(32, 128) <= cus                                         ? 1
                                                                                      : 2;

@@ -69,7 +69,9 @@ __device__ __forceinline__ void q8w_widen4(uint32_t w, uint32_t &lo, uint32_t &h
 // banks), double-buffered. The 16-deep steps rotate over NACC sets of accumulators, added in
 // order at the end: shorter sums, and MFMAs that do not wait for the one before.
 // W: the fragment-major image of an Np x Kp weight (Kp a multiple of 64, Np of BN); ws[N].
-// VEC: lda % 4 == 0, K % 4 == 0 and A 16-byte aligned (16-byte loads).
+// VEC: lda % 4 == 0, K % 4 == 0 and A 16-byte aligned (16-byte loads). Otherwise the chunks inside
+// K load the same 16 bytes at 4-byte alignment, and the last one value by value (all of them did for
+// a while: 8192 x 4096, K = 2047 417 us, 358 so; 4000 x 1000, K = 1001 53 and 38).
 // What bounds it: with a block or two per CU the serial latency of a chunk, hence 32-row tiles
 // and deep chunks; with many tiles the MFMA and the splitting's VALU work. Measured on MI355X
 // against the form before (64 x 64 to 128 x 256 tiles, 32-deep chunks, branches around the
@@ -103,6 +105,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_q8w(
     u32x4 wr[KB][TN];
     auto load_a = [&](int c) {
         const int k = KC * c + lk;
+        if (!VEC && KC * c + KC <= K) {  // uniform: all of the chunk, in unaligned 16-byte loads
+#pragma unroll
+            for (int i = 0; i < AV; ++i) ra[i] = f32x4{ga[i][k], ga[i][k + 1], ga[i][k + 2], ga[i][k + 3]};
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < AV; ++i) {
             if (VEC) ra[i] = *reinterpret_cast<const f32x4 *>(ga[i] + min(k, K - 4));
