@@ -109,7 +109,8 @@ def test_the_scratch_grows_while_in_use(shared):
 def test_another_stream_waits_for_the_scratch_alone():
     # The context's stream: a linear (it uses the scratch), then f32 products of some 100 ms (they do
     # not). A linear on another stream, once such a stream has used the scratch before, waits for the
-    # first linear and not for the products.
+    # first linear and not for the products. (Streams share a few hardware queues, and work on one
+    # queue runs in order: of several streams, one that has a queue of its own shows it.)
     import torch
 
     g = workloads.rng(32)
@@ -119,7 +120,6 @@ def test_another_stream_waits_for_the_scratch_alone():
         a = torch.from_numpy(workloads.activations(g, M, K)).cuda()
         big = torch.randn((8192, 8192), device="cuda")
         out, prod = torch.empty((M, N), device="cuda"), torch.empty((8192, 8192), device="cuda")
-        s = torch.cuda.Stream()
         torch.cuda.synchronize()
 
         def linear(stream):
@@ -130,13 +130,20 @@ def test_another_stream_waits_for_the_scratch_alone():
                 c.matmul_bt_f32_dev(big.data_ptr(), 8192, big.data_ptr(), 8192, enchip.B_NK, prod.data_ptr(), 8192, 8192,
                                     8192, 8192)
 
-        linear(0), products(1), linear(s.cuda_stream)  # kernels loaded, the other stream known
+        linear(0), products(1)  # kernels loaded
         torch.cuda.synchronize()
-        print("[case] scratch order beside f32 products", flush=True)
-        linear(0), products(30), linear(s.cuda_stream)
-        t0 = time.perf_counter()
-        s.synchronize()
-        t1 = time.perf_counter()
-        torch.cuda.synchronize()
-        t2 = time.perf_counter()
-        assert t1 - t0 < (t2 - t0) / 4, f"the other stream ended after {t1 - t0:.4f} of {t2 - t0:.4f} s"
+        shares = []
+        for i in range(8):
+            s = torch.cuda.Stream()
+            linear(0), linear(s.cuda_stream)  # such a stream has used the scratch
+            torch.cuda.synchronize()
+            print(f"[case] scratch order beside f32 products, stream {i}", flush=True)
+            linear(0), products(30), linear(s.cuda_stream)
+            t0 = time.perf_counter()
+            s.synchronize()
+            t1 = time.perf_counter()
+            torch.cuda.synchronize()
+            shares.append((t1 - t0) / (time.perf_counter() - t0))
+            if shares[-1] < 0.25:
+                return
+        raise AssertionError(f"the other streams waited for {shares} of the products")
