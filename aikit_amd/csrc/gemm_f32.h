@@ -11,10 +11,11 @@
 //
 // Arithmetic. Every operand value is split into three bf16 parts, x = h + m + l (h
 // the bf16 nearest x, m the one nearest x - h, l the rest, which has at most 8 bits), and a
-// product is the six products of parts above 2^-25 of it: h.h', h.m', m.h', m.m', h.l', l.h',
-// each exact on v_mfma_f32_32x32x16_bf16 and summed in f32. The three left out, m.l', l.m'
-// and l.l', are within 2^-26 |x y|, an eighth of what rounding the sum once costs, and a
-// 16-deep step rounds the sum 6 times where the f32 MFMA (32x32x2) rounds it 8 to 16 times.
+// product is six products of parts: h.h', h.m', m.h', m.m', h.l', l.h', each exact on
+// v_mfma_f32_32x32x16_bf16 and summed in f32. The three left out, m.l', l.m' and l.l', come to at
+// most 2^-24 |x y| (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|; typically under 2^-26), what rounding the
+// product once costs, and a 16-deep step rounds the sum 6 times where the f32 MFMA (32x32x2) rounds
+// it 8 to 16 times.
 // Measured against float64 (standard normal operands, relative 2-norm): K = 768 4.2e-7, or
 // 2.1e-7 with K split over wavefronts, against the f32 MFMA's 5.0e-7; K = 3072 8.7e-7 /
 // 4.3e-7 against 9.9e-7. The contract is the reference's gate against a float64 dot product

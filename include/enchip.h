@@ -23,7 +23,8 @@
  *   - The context's device scratch (the quantized activations of the entry points
  *     that quantize themselves, the top-k candidates) is shared by all of them. Work
  *     that uses it on one stream waits, on the device, for its last use on another
- *     stream (through an event of the library), so host calls and
+ *     stream (through an event of the library; the first work on a caller's stream waits
+ *     for all that the context's stream holds), so host calls and
  *     *_dev calls on different streams may be mixed. Under HIP graph capture the
  *     library records no such event and the caller orders the streams.
  *
@@ -282,10 +283,14 @@ int enchip_probe_ceilings(enchip_ctx *ctx, enchip_ceilings *out);
  * encoder.Backend.MatmulBT (encoder/backend.go:19-28; enccuda's MatmulBT,
  * gpu/enccuda/backend.go:136-172). Synchronous. a and b are uploaded on every call
  * (their contents are never cached: attention rewrites the same pooled buffers
- * between calls), dst is downloaded before returning. Products and sums are f32 on
- * the f32 MFMA in an order of its own; the contract is the reference's gate, worst
- * |dst - float64 dot| / max(|float64 dot|, 1) <= 2e-4 (gpu/enccuda/backend_test.go:
- * 47-86). K == 0 gives zeros. Which shapes are worth the round trip is the caller's
+ * between calls), dst is downloaded before returning. Every operand is split into three
+ * bf16 parts and six of their products are summed in f32 on the bf16 MFMA, in an order of
+ * its own; infinities, NaN, sums that overflow, and outputs that operands under 2^-110
+ * matter to are computed on the f32 MFMA, over the whole range of f32. The error against
+ * float64 is no larger than f32 products' would be; the contract is the reference's gate,
+ * worst |dst - float64 dot| / max(|float64 dot|, 1) <= 2e-4 (gpu/enccuda/backend_test.go:
+ * 47-86). An output does not depend on the batch, the pitch or the values of other rows and columns.
+ * K == 0 gives zeros. Which shapes are worth the round trip is the caller's
  * choice (enccuda's minGPUFlops, gpu/enccuda/backend.go:48-75): this entry point
  * always runs on the device. */
 int enchip_matmul_bt_f32(enchip_ctx *ctx, const float *a, const float *b, float *dst,

@@ -18,7 +18,7 @@ SHAPES = [(33, 300, 132, "k32"), (500, 257, 1000, "k64x32"), (1, 1024, 4097, "k"
 
 def bound(a, b, K):
     """|C - exact| <= (adds + 2) 2^-24 sum |a b|: 6 rounded adds of the running sum per 16-deep
-    step, the K split's 3 and the products left out (under 2^-25 each)."""
+    step, the K split's 3 and the products left out (together under 2^-24 |a b|)."""
     return (6 * -(-K // 16) + 3 + 2) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T)
 
 
