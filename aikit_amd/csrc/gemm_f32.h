@@ -114,7 +114,7 @@ __device__ __forceinline__ bool any_nonfinite(const f32x16 (&acc)[TM][TN], float
         for (int t = 0; t < TN; ++t)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                s += acc[i][t][e] * 0.0f;
+                s = __builtin_fmaf(acc[i][t][e], 0.0f, s);
                 least = fminf(fabsf(acc[i][t][e]), least);
             }
     return s != 0.0f;  // 0, or NaN
@@ -403,18 +403,18 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_tile(
         for (int s = 0; s < KC / 16; ++s) mfma_parts<TM, TN>(pa[s], pb[s], acc);
         lds_barrier();
     }
-    // The last loads, of a chunk already used, end here: left in flight, their registers' next use
-    // waits in each store's branch, for the stores before it too (16 x 64 problems 3.6 -> 4.1 us).
-#pragma unroll
-    for (int i = 0; i < AV; ++i) asm volatile("" ::"v"(ra[i]));
-#pragma unroll
-    for (int i = 0; i < BV; ++i) asm volatile("" ::"v"(rb[i]));
     if (big > kBig) any_big = 1;
     lds_barrier();
     float least = INFINITY;
     const bool nonfinite = __builtin_amdgcn_ballot_w64(any_nonfinite<TM, TN>(acc, least)) != 0;
     const bool low = __builtin_amdgcn_ballot_w64(least < lost_below(K)) != 0;
     const int m0 = bm0 + 32 * TM * wm, n0 = bn0 + 32 * TN * wn;
+    // The last loads, of a chunk already used, end here: left in flight, their registers' next use
+    // waits in each store's branch, for the stores before it too (16 x 64 problems 3.6 -> 4.1 us).
+#pragma unroll
+    for (int i = 0; i < AV; ++i) asm volatile("" ::"v"(ra[i]));
+#pragma unroll
+    for (int i = 0; i < BV; ++i) asm volatile("" ::"v"(rb[i]));
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
